@@ -122,6 +122,7 @@ inline size_t tiled_weight_count(const bf_dims& d) {   // formats.hpp:58-61
 
 // ------------------------------------------------------------ device side
 typedef _Float16 bf_half8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf_bfloat8 __attribute__((ext_vector_type(8)));
 typedef float bf_float4 __attribute__((ext_vector_type(4)));
 typedef int bf_int4v __attribute__((ext_vector_type(4)));
 typedef unsigned int bf_uint4v __attribute__((ext_vector_type(4)));
@@ -153,5 +154,18 @@ __device__ __forceinline__ void bf_int4x4_to_half2x4(unsigned d, unsigned out[4]
         const h2 bias = {(_Float16)1032.0f, (_Float16)1032.0f};
         v = v - bias;
         out[j] = __builtin_bit_cast(unsigned, v);
+    }
+}
+
+// The same into bfloat16 pairs: an integer of [-8, 7] has its float value in
+// the upper 16 bits.
+__device__ __forceinline__ void bf_int4x4_to_bfloat2x4(unsigned d, unsigned out[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float re = (float)bf_nibble(d, 8 * j);
+        const float im = (float)bf_nibble(d, 8 * j + 4);
+        // (upper half of re, upper half of im)
+        out[j] = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, im),
+                                       __builtin_bit_cast(unsigned, re), 0x07060302u);
     }
 }

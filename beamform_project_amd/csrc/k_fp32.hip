@@ -1,4 +1,6 @@
-// k_fp32.hip -- plain FP32 fused fixed-grid beamformer for gfx950.
+// k_fp32.hip -- the fixed-grid beamformer with float weights for gfx950: most
+// calls go to the matrix cores (k_mfma_exact.hip); the FMA kernel here takes
+// the small ones and the window lengths that kernel does not have.
 //
 // out[w][f][b] = sum_{t in window w} | sum_a W[b][f][a] * X[t][f][a] |^2
 // (no conjugate, reference src/cpu_beamformer.cpp:56-78 and the integration
@@ -12,7 +14,7 @@
 // 4 FMAs per complex MAC for each of its BB beams.  Windows longer than one
 // lane's share are split over P adjacent lanes and folded with a butterfly
 // of cross-lane adds.
-#include "bf_kernels.hpp"
+#include "mfma_fused.hpp"
 
 namespace bfhip {
 namespace {
@@ -137,6 +139,21 @@ void launch_a(hipStream_t stream, const uint8_t* x, const float* w, bool tiled, 
 void launch_fp32_fused(hipStream_t stream, const uint8_t* x, const float* w,
                        WeightLayout layout, float* out, size_t T, size_t F, size_t A,
                        size_t B, size_t S) {
+    // On the matrix cores with the float weights in three exact slices where
+    // that is faster: from four beams (eight share a tile column block) once
+    // the call is not launch-bound, and for fewer beams in long calls, where
+    // the FMA kernel's lanes each walk a whole window alone (A = 64, T = 8192:
+    // B = 2, S = 320 351 -> 97 us, B = 40 747 -> 176 us, B = 128 2294 -> 362 us;
+    // but A = 256, T = 320, B = 1 18 -> 36 us, A = 256, T = 64, B = 3 11 -> 15 us
+    // and A = 32, T = 8192, B = 2, S = 0 65 -> 83 us, which stay on FMAs).
+    const bool pays = B >= 4 ? T * B * A >= 65536 : T >= 2048 && (S > 0 || A > 32);
+    if (pays && mfma_supported(A, B, S) && T <= (size_t)INT32_MAX / 8 && S <= (size_t)INT32_MAX / 8 &&
+        F <= 65535) {
+        const MfmaLaunch L{x, w, out, nullptr, (int)T, (int)F, (int)B, (int)S, 3,
+                           layout == WeightLayout::Tiled};
+        launch_mfma_exact(stream, L, (int)A);
+        return;
+    }
     // S == 0: one "window" per spectrum.
     const size_t s_eff = S == 0 ? 1 : S;
     const size_t W = ceil_div(T, s_eff);

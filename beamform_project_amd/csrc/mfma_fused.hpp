@@ -6,10 +6,11 @@
 //   [xr0 xi0 xr1 xi1 ...] (1 x 2A)  *  B (2A x 2B),
 // where output column 2b holds Re(y_b) (weights (wr, -wi) per antenna) and
 // column 2b+1 holds Im(y_b) (weights (wi, wr)).  int4 samples are exact in
-// FP16, so the only rounding in the products comes from the weights: the
-// SPLIT variant stores each weight as hi = fp16(w) plus lo = fp16(w - hi)
-// and runs the K loop twice over the same A operand (products are exact in
-// the FP32 accumulator), recovering ~22 significant bits per weight.
+// FP16 (and in bfloat16), so the only rounding in the products comes from
+// the weights, which are held in PARTS slices: one fp16; hi = fp16(w) plus
+// lo = fp16(w - hi), ~22 significant bits; or three bfloat16, the float
+// itself.  The K loop runs over every slice with the same A operand
+// (products are exact in the FP32 accumulator).
 //
 // Instruction: v_mfma_f32_16x16x32_f16.  A workgroup of WV waves owns one
 // frequency, one chunk of time and WV*NT*8 beams; each wave keeps the
@@ -35,6 +36,11 @@
 //   MODE 0 (no integration): tile i, row 4G+r -> t = 16i + 4G + r
 //   MODE 1 (S == 10): super-tile of 5 tiles, G covers 20 spectra (2 windows)
 //   MODE 2 (S % 4 == 0): super-tile of S/4 tiles, G covers one window
+//   MODE 3 (S % 64 == 0): tiles as in MODE 0; the row groups share every
+//     window and are folded by two shuffles where it closes.  Windows are
+//     this long that a stage of 4 tiles lies inside one, and the work is
+//     whole windows, not groups of four (A = 256, T = 4100, B = 45, S = 320, 13
+//     windows: 437 -> 383 us)
 // Re and im of a beam sit in adjacent lanes; a quad-permute DPP adds the
 // two squared sums.
 #pragma once
@@ -52,7 +58,8 @@ struct MfmaLaunch {
     float* out = nullptr;
     const uint8_t* mask = nullptr;  // [T][F] frame validity (0 = lost), or null
     int T = 0, F = 0, B = 0, S = 0;
-    bool split = true;
+    int parts = 2;       // weight slices: 1 fp16, 2 fp16 hi + lo, 3 bfloat16 (the float itself)
+    bool tiled = false;  // weights [F][B/32][A][32] instead of [B][F][A]
 };
 
 // Launch the kernel of `cfg` for one antenna count; false when `cfg` is
@@ -73,53 +80,100 @@ __device__ __forceinline__ float dpp_swap_pairs(float v) {
         float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
 }
 
-// Loads the B operand (weights) of one wave into registers.
-template <int A, int NT, bool SPLIT>
-__device__ __forceinline__ void load_weights(const float2* __restrict__ w, int F, int B,
-                                             int f, int beam0, int lane,
-                                             bf_half8 (&bhi)[NT][A / 16],
-                                             bf_half8 (&blo)[NT][A / 16]) {
+// PARTS names how a weight reaches the matrix unit: 1 = fp16(w); 2 = fp16
+// hi + lo, about 22 bits; 3 = three bfloat16 slices of 8 bits each, which
+// together are the float weight itself (bfloat16 has float's exponent), so
+// every product with an int4 sample is exact and only the FP32 accumulation
+// rounds.
+template <int PARTS>
+__device__ __forceinline__ bf_float4 mfma_16x16x32(bf_half8 a, bf_half8 b, bf_float4 c) {
+    if constexpr (PARTS == 3)
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf_bfloat8, a),
+                                                       __builtin_bit_cast(bf_bfloat8, b), c, 0, 0,
+                                                       0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+// Slice q of the weight component e, as the 16 bits of its operand element.
+// Bfloat16 slices are cut off, not rounded: 8 + 8 + 8 bits hold all 24 of
+// a float.  Infinities and NaN stay whole in slice 0.
+template <int PARTS>
+__device__ __forceinline__ void weight_slices(float e, _Float16 (&out)[PARTS]) {
+    if constexpr (PARTS == 3) {
+        auto top = [](float v) { return __builtin_bit_cast(unsigned, v) & 0xFFFF0000u; };
+        auto bits = [](unsigned u) {
+            return __builtin_bit_cast(_Float16, (unsigned short)(u >> 16));
+        };
+        unsigned h = top(e);
+        float r = e - __builtin_bit_cast(float, h);
+        if (!isfinite(e)) {
+            r = 0.0f;
+            if (isnan(e)) h |= 0x00400000u;  // a NaN of low payload bits only stays a NaN
+        }
+        const unsigned m = top(r);
+        out[0] = bits(h);
+        out[1] = bits(m);
+        out[2] = bits(top(r - __builtin_bit_cast(float, m)));
+    } else {
+        out[0] = (_Float16)e;
+        if constexpr (PARTS == 2) out[1] = (_Float16)(e - (float)out[0]);
+    }
+}
+
+// Loads the B operand (weights) of one wave into registers: canonical
+// [B][F][A], or tiled [F][B/32][A][32].
+template <int A, int NT, int PARTS>
+__device__ __forceinline__ void load_weights(const float2* __restrict__ w, bool tiled, int F,
+                                             int B, int f, int beam0, int lane,
+                                             bf_half8 (&bw)[PARTS][NT][A / 16]) {
     constexpr int KS = A / 16;
     const int c = lane & 15;
     const int g = lane >> 4;
+    const int tiles = (B + 31) / 32;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         const int b = beam0 + nt * 8 + (c >> 1);
         const bool comp_im = (c & 1) != 0;
+        const float2* const wb = tiled ? w + ((size_t)f * tiles + b / 32) * A * 32 + b % 32
+                                       : w + ((size_t)b * F + f) * A;
+        const int step = tiled ? 32 : 1;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-            bf_half8 h, l;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int a = g * (A / 4) + 4 * s + j;
                 float2 v = make_float2(0.0f, 0.0f);
-                if (b < B) v = w[((size_t)b * F + f) * A + a];
+                if (b < B) v = wb[a * step];
                 // column re: (wr, -wi); column im: (wi, wr)
-                const float e0 = comp_im ? v.y : v.x;
-                const float e1 = comp_im ? v.x : -v.y;
-                const _Float16 h0 = (_Float16)e0;
-                const _Float16 h1 = (_Float16)e1;
-                h[2 * j] = h0;
-                h[2 * j + 1] = h1;
-                if (SPLIT) {
-                    l[2 * j] = (_Float16)(e0 - (float)h0);
-                    l[2 * j + 1] = (_Float16)(e1 - (float)h1);
+                _Float16 e0[PARTS], e1[PARTS];
+                weight_slices<PARTS>(comp_im ? v.y : v.x, e0);
+                weight_slices<PARTS>(comp_im ? v.x : -v.y, e1);
+#pragma unroll
+                for (int q = 0; q < PARTS; ++q) {
+                    bw[q][nt][s][2 * j] = e0[q];
+                    bw[q][nt][s][2 * j + 1] = e1[q];
                 }
             }
-            bhi[nt][s] = h;
-            if (SPLIT) blo[nt][s] = l;
         }
     }
 }
 
 // At least two waves per SIMD (at most 256 registers per lane): the
 // unrolled stage otherwise keeps several tiles' accumulators in flight.
-template <int A, int NT, int WV, bool SPLIT, int MODE, int ST, bool DB, bool MASKED = false>
-__global__ __launch_bounds__(WV * kWaveSize) __attribute__((amdgpu_waves_per_eu(2)))
+// Eight-wave groups with 64 registers of weights and one LDS stage run two
+// to a CU within 128 registers (1.02 ms against 1.30 ms at A = 64, T = 32768,
+// B = 128, S = 10 where six registers more leave one group).
+constexpr int min_waves(int A, int NT, int WV, int parts, bool db) {
+    return WV == 8 && !db && parts * NT * A / 4 == 64 ? 4 : 2;
+}
+template <int A, int NT, int WV, int PARTS, int MODE, int ST, bool DB, bool MASKED = false>
+__global__ __launch_bounds__(WV * kWaveSize)
+__attribute__((amdgpu_waves_per_eu(min_waves(A, NT, WV, PARTS, DB))))
 void mfma_fused_kernel(
-    const uint8_t* __restrict__ x, const float2* __restrict__ w, float* __restrict__ out,
-    const uint8_t* __restrict__ mask, int T, int F, int B, int S, int W, int tiles_total,
-    int tiles_per_chunk, int n_items, int per_xcd) {
+    const uint8_t* __restrict__ x, const float2* __restrict__ w, bool tiled,
+    float* __restrict__ out, const uint8_t* __restrict__ mask, int T, int F, int B, int S, int W,
+    int tiles_total, int tiles_per_chunk, int n_items, int per_xcd) {
     constexpr int kThreads = WV * kWaveSize;
     constexpr int KS = A / 16;                      // k-steps of 32 (16 antennas x re/im)
     using Map = StageMap<A, kThreads>;
@@ -151,16 +205,16 @@ void mfma_fused_kernel(
     const int beam0 = (blockIdx.y * WV + wave) * NT * 8;
     const bool has_beams = beam0 < B;
 
-    bf_half8 bhi[NT][KS];
-    bf_half8 blo[NT][KS];
-    if (has_beams) load_weights<A, NT, SPLIT>(w, F, B, f, beam0, lane, bhi, blo);
+    bf_half8 bw[PARTS][NT][KS];
+    if (has_beams) load_weights<A, NT, PARTS>(w, tiled, F, B, f, beam0, lane, bw);
 
     const int tile_begin = chunk * tiles_per_chunk;
     int tile_end = tile_begin + tiles_per_chunk;
     tile_end = tile_end < tiles_total ? tile_end : tiles_total;
     const size_t row_stride = (size_t)F * A;
-    const int tps = MODE == 2 ? (S >> 2) : 5;           // tiles per super-tile
-    const int pitch = MODE == 0 ? 4 : (MODE == 1 ? 20 : S);  // spectra between row groups
+    // tiles per super-tile (MODE 3: per window)
+    const int tps = MODE == 2 ? (S >> 2) : (MODE == 3 ? (S >> 4) : 5);
+    const int pitch = MODE == 0 || MODE == 3 ? 4 : (MODE == 1 ? 20 : S);  // spectra between row groups
 
     // Per-thread staging constants (StageMap: rows fastest within 16 lanes).
     const int tl0 = Map::tile0(wave);  // uniform per wave
@@ -175,11 +229,11 @@ void mfma_fused_kernel(
     // First spectrum of the stage starting at tile st0, and offset of tile
     // tl of a stage from it (row group 0, row 0).
     auto stage_time = [&](int st0) -> int {
-        if (MODE == 0 || MODE == 1) return 16 * st0;  // MODE 1: 80 per super-tile
+        if (MODE != 2) return 16 * st0;  // MODE 1: 80 per super-tile
         return 4 * S * (st0 / tps) + 4 * (st0 % tps);
     };
     auto tile_rows = [&](int tl) -> int {
-        if (MODE == 0) return 16 * tl;
+        if (MODE == 0 || MODE == 3) return 16 * tl;
         if (MODE == 1) return ST == 5 ? 4 * tl : 80 * (tl / 5) + 4 * (tl % 5);
         return 4 * tl;
     };
@@ -211,7 +265,10 @@ void mfma_fused_kernel(
     auto store_dword = [&](int k, unsigned char* buf) {
         if (!dword_valid(k)) return;
         unsigned h2[4];
-        bf_int4x4_to_half2x4(pre[k], h2);
+        if (PARTS == 3)
+            bf_int4x4_to_bfloat2x4(pre[k], h2);
+        else
+            bf_int4x4_to_half2x4(pre[k], h2);
         bf_uint4v u = {h2[0], h2[1], h2[2], h2[3]};
         *reinterpret_cast<bf_uint4v*>(buf + lds_mine + Map::lds_delta(k)) = u;
     };
@@ -240,6 +297,7 @@ void mfma_fused_kernel(
     float* const out_lane =
         MODE == 1 ? out + ((size_t)(2 * G + odd) * F + f) * B + bl
         : MODE == 2 ? out + ((size_t)G * F + f) * B + bl + (NT >= 2 ? 8 * odd : 0)
+        : MODE == 3 ? out + (size_t)f * B + bl
                     : out + ((size_t)(4 * G + odd) * F + f) * B + bl;
     const size_t group_stride = (size_t)F * B;  // floats between consecutive windows
 
@@ -319,11 +377,24 @@ void mfma_fused_kernel(
                 for (int nt = 0; nt < NT; nt += 2)
                     if (ok && bl + (nt + odd) * 8 < B) o[nt * 8] = odd ? p[nt + 1] : p[nt];
             }
+        } else if (MODE == 3) {
+            float* const o = out_lane + (size_t)(i0 / tps) * group_stride;
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                float p = win[nt][0];
+                p += __shfl_xor(p, 16);
+                p += __shfl_xor(p, 32);
+                p += dpp_swap_pairs(p);
+                win[nt][0] = 0.0f;
+                if (G == nt % 4 && !odd && bl + nt * 8 < B) o[nt * 8] = p;
+            }
         }
     };
-    // MODE 2: whether the stage at st0 ends a super-tile (MODE 1 closes
-    // its windows inside the stage, after every fifth tile).
+    // MODE 2, 3: whether the stage at st0 ends a super-tile or window (MODE
+    // 1 closes its windows inside the stage, after every fifth tile).  The
+    // last window may be cut short by T.
     auto closes_window = [&](int st0) -> bool {
+        if (MODE == 3) return (st0 % tps) + ST == tps || st0 + ST >= tiles_total;
         return MODE == 2 && (st0 % tps) + ST == tps;
     };
 
@@ -364,15 +435,10 @@ void mfma_fused_kernel(
                                  : *reinterpret_cast<const bf_half8*>(
                                        cur + tl * TILE_BYTES + (s * kWaveSize + lane) * 16);
 #pragma unroll
-                    for (int nt = 0; nt < NT; ++nt)
-                        acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_s, bhi[nt][s],
-                                                                         acc[nt], 0, 0, 0);
-                    if (SPLIT) {
+                    for (int q = 0; q < PARTS; ++q)
 #pragma unroll
                         for (int nt = 0; nt < NT; ++nt)
-                            acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_s, blo[nt][s],
-                                                                             acc[nt], 0, 0, 0);
-                    }
+                            acc[nt] = mfma_16x16x32<PARTS>(a_s, bw[q][nt][s], acc[nt]);
                 }
             }
             if (DB) {
@@ -451,7 +517,7 @@ struct Plan {
 
 inline Plan make_plan(int T, int F, int B, int S, const MfmaConfig& cfg) {
     Plan p{};
-    p.mode = S == 0 ? 0 : (S == 10 ? 1 : 2);
+    p.mode = S == 0 ? 0 : (S == 10 ? 1 : (S % 64 == 0 ? 3 : 2));
     int tiles_per_super = 1;
     if (p.mode == 0) {
         p.st = 4;
@@ -460,15 +526,20 @@ inline Plan make_plan(int T, int F, int B, int S, const MfmaConfig& cfg) {
         p.st = 5;
         tiles_per_super = 5;
         p.W = (int)ceil_div((size_t)T, 10);
+    } else if (p.mode == 3) {
+        p.st = 4;
+        tiles_per_super = S / 16;
+        p.W = (int)ceil_div((size_t)T, (size_t)S);
     } else {
         tiles_per_super = S / 4;
-        p.st = tiles_per_super % 4 == 0 ? 4 : 1;
+        p.st = tiles_per_super % 4 == 0 ? 4 : (tiles_per_super % 5 == 0 ? 5 : 1);
         p.W = (int)ceil_div((size_t)T, (size_t)S);
     }
     const int rows_super = 16 * tiles_per_super;
     const int n_super = (int)ceil_div((size_t)T, (size_t)rows_super);
     p.tiles_total = n_super * tiles_per_super;
-    if (p.mode == 0) p.tiles_total = (int)ceil_div((size_t)p.tiles_total, 4) * 4;
+    // tiles in time order: whole stages up to T
+    if (p.mode == 0 || p.mode == 3) p.tiles_total = 4 * (int)ceil_div((size_t)T, 64);
     p.beam_blocks = (int)ceil_div((size_t)B, (size_t)(cfg.waves * cfg.nt * 8));
     // Chunk length: a whole number of super-tiles and stages, chosen to
     // minimise (rounds of resident workgroups) x (tiles per workgroup + a
@@ -495,23 +566,27 @@ inline Plan make_plan(int T, int F, int B, int S, const MfmaConfig& cfg) {
     return p;
 }
 
-template <int A, int NT, int WV, bool SPLIT, bool DB, bool MASKED = false>
+template <int A, int NT, int WV, int PARTS, bool DB, bool MASKED = false>
 void launch_shape(hipStream_t stream, const MfmaLaunch& L, const MfmaConfig& cfg) {
     const Plan p = make_plan(L.T, L.F, L.B, L.S, cfg);
     const dim3 grid((unsigned)(p.per_xcd * kXcds), (unsigned)p.beam_blocks);
     const dim3 block(WV * kWaveSize);
     const float2* w2 = reinterpret_cast<const float2*>(L.w);
 #define BF_LAUNCH(MODE_, ST_)                                                                 \
-    hipLaunchKernelGGL((mfma_fused_kernel<A, NT, WV, SPLIT, MODE_, ST_, DB, MASKED>), grid,   \
+    hipLaunchKernelGGL((mfma_fused_kernel<A, NT, WV, PARTS, MODE_, ST_, DB, MASKED>), grid,   \
                        block, 0,                                                               \
-                       stream, L.x, w2, L.out, L.mask, L.T, L.F, L.B, L.S, p.W, p.tiles_total, \
-                       p.tiles_per_chunk, p.n_items, p.per_xcd)
+                       stream, L.x, w2, L.tiled, L.out, L.mask, L.T, L.F, L.B, L.S, p.W,       \
+                       p.tiles_total, p.tiles_per_chunk, p.n_items, p.per_xcd)
     if (p.mode == 0) {
         BF_LAUNCH(0, 4);
     } else if (p.mode == 1) {
         BF_LAUNCH(1, 5);
+    } else if (p.mode == 3) {
+        BF_LAUNCH(3, 4);
     } else if (p.st == 4) {
         BF_LAUNCH(2, 4);
+    } else if (p.st == 5) {
+        BF_LAUNCH(2, 5);
     } else {
         BF_LAUNCH(2, 1);
     }
@@ -520,20 +595,24 @@ void launch_shape(hipStream_t stream, const MfmaLaunch& L, const MfmaConfig& cfg
 
 template <int A, int NT, int WV>
 void launch_split_db(hipStream_t stream, const MfmaLaunch& L, const MfmaConfig& cfg) {
-    if (L.split) {
+    if (L.parts == 2) {
         if (cfg.db)
-            launch_shape<A, NT, WV, true, true>(stream, L, cfg);
+            launch_shape<A, NT, WV, 2, true>(stream, L, cfg);
         else
-            launch_shape<A, NT, WV, true, false>(stream, L, cfg);
+            launch_shape<A, NT, WV, 2, false>(stream, L, cfg);
     } else {
         if (cfg.db)
-            launch_shape<A, NT, WV, false, true>(stream, L, cfg);
+            launch_shape<A, NT, WV, 1, true>(stream, L, cfg);
         else
-            launch_shape<A, NT, WV, false, false>(stream, L, cfg);
+            launch_shape<A, NT, WV, 1, false>(stream, L, cfg);
     }
 }
 
 }  // namespace mfma_detail
+
+// Launches the kernel with float weights (PARTS = 3) for `A` antennas
+// (k_mfma_exact.hip): `L.tiled` chooses the weight layout.
+void launch_mfma_exact(hipStream_t stream, const MfmaLaunch& L, int A);
 
 // Instantiated shapes per antenna count: (NT, waves) pairs whose split
 // weights fit in at most 128 VGPRs per lane and that compile without
@@ -553,10 +632,10 @@ void launch_split_db(hipStream_t stream, const MfmaLaunch& L, const MfmaConfig& 
             m.nt = 1;                                                                      \
             m.waves = 4;                                                                   \
             m.db = 0;                                                                      \
-            if (L.split)                                                                   \
-                mfma_detail::launch_shape<A_, 1, 4, true, false, true>(stream, L, m);      \
+            if (L.parts == 2)                                                              \
+                mfma_detail::launch_shape<A_, 1, 4, 2, false, true>(stream, L, m);      \
             else                                                                           \
-                mfma_detail::launch_shape<A_, 1, 4, false, false, true>(stream, L, m);     \
+                mfma_detail::launch_shape<A_, 1, 4, 1, false, true>(stream, L, m);         \
             return true;                                                                   \
         }                                                                                  \
         SHAPES                                                                             \
