@@ -41,7 +41,7 @@ COMMON_FLAGS = [
 # (bit-exact parity with the reference CPU code): no a*b+c contraction.
 PER_FILE_FLAGS = {
     "k_quant.hip": ["-ffp-contract=off"],
-    "k_tracker.hip": ["-ffp-contract=off"],
+    **{f"k_tracker{v}.hip": ["-ffp-contract=off"] for v in ("", "_a32", "_a64", "_a128", "_a256")},
     "k_opt_tracker.hip": ["-ffp-contract=off"],
 }
 

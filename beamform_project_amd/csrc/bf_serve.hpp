@@ -6,8 +6,7 @@
 // and a control block.  A step processes every window of every active slot
 // whose last spectrum lies in (previous head, head]: a one-workgroup plan
 // kernel reads the step's head and turns the slot table into work offsets,
-// and one persistent kernel works through workgroup items (multi-tile
-// windows) and then wave tasks (one-tile windows).
+// and one persistent kernel works through the wave tasks.
 #pragma once
 
 #include "bf_tracker.hpp"
@@ -29,7 +28,7 @@ struct ServeSlot {
     int active;
     int B;
     int S;
-    int wpi;  // windows per work item
+    int wpi;  // windows per wave task
     long long t0;
     long long t_end;
     long long out_windows;
@@ -53,17 +52,14 @@ struct ServeCtrl {
 // flight, so an entry is never rewritten before its step has read it.
 inline constexpr int kServeHeadRing = 4096;
 
-// Windows of one wave task of a one-tile-window slot.
-inline constexpr int kServeShortRun = 16;
+// Beams of one wave task.
+inline constexpr int kServeTaskBeams = 16;
 
-// Per-step work table written by the plan kernel.  Slots whose windows span
-// several 16-spectrum tiles make workgroup items (run of windows, channel),
-// [off_long[s], off_long[s+1]); slots whose windows fit one tile make wave
-// tasks (run of up to kServeShortRun windows, 16-beam block, channel),
-// [off_short[s], off_short[s+1]).  Channels are fastest in both.
+// Per-step work table written by the plan kernel.  Slot s makes the wave
+// tasks [off[s], off[s+1]): (run of wpi windows, channel, block of
+// kServeTaskBeams beams), blocks fastest, then channels.
 struct ServeWork {
-    int off_long[kServeMaxSlots + 1];
-    int off_short[kServeMaxSlots + 1];
+    int off[kServeMaxSlots + 1];
     int w_lo[kServeMaxSlots];
     int n_win[kServeMaxSlots];
 };
@@ -82,7 +78,7 @@ struct ServeLaunch {
     bool split = true;
 };
 
-// Windows per workgroup item for multi-tile windows (about 16 tiles).
+// Windows per wave task (about 16 tiles of 16 spectra).
 inline int serve_windows_per_item(int S) {
     const int tpw = (S + 15) / 16;
     const int w = 16 / tpw;

@@ -1,0 +1,98 @@
+"""The multi-beam tracker's wave body and its steering weights at the sizes
+where they can go wrong: windows around the tile of 16 spectra and the groups
+of four tiles, runs of anchored windows, beams around the 8-beam columns and
+the blocks of 16 and 32, few and many channels, baselines beyond the phase's
+integer form, and directions that leave the sky.
+
+Bars as in test_gpu_tracker.py: 1e-5 floored against FP64 for split-FP16 and
+float weights, 2e-3 for single FP16.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+from beamform_project_amd import api
+from beamform_project_amd import tracker as TR
+from helpers import incoherent_floor, rel_err_floored
+
+pytestmark = pytest.mark.gpu
+
+K = api.Kernel
+KERNELS = ((K.SPLIT_F16, 1e-5), (K.F16, 2e-3), (K.FP32, 1e-5))
+
+
+def case(T, F, A, B, S, seed, step=1e-3, scale=0.3):
+    """Directions that move by up to `step` per window."""
+    rng = np.random.default_rng(seed)
+    x = O.make_uniform_int4(T * F * A, seed).reshape(T, F, A)
+    pos = O.regular_array(A // 8, 8, 0.3) * np.float32(scale / 0.3)
+    pos[:, 2] = rng.uniform(-1, 1, A) * scale
+    fr = np.linspace(400e6, 800e6, F).astype(np.float32)
+    W = -(-T // S)
+    lm = rng.uniform(-0.4, 0.4, (B, 2)) + np.arange(W)[:, None, None] * \
+        rng.uniform(-step, step, (B, 2))
+    lm = np.clip(lm, -0.6, 0.6)
+    dirs = np.concatenate([lm, np.sqrt(1 - (lm ** 2).sum(-1, keepdims=True))], -1)
+    return x, pos, fr, np.ascontiguousarray(dirs, np.float32)
+
+
+def launch(x, pos, fr, dirs, T, F, A, B, S, integrate, kernel):
+    arrays = [api.DeviceArray.from_numpy(a) for a in (x, pos, fr, dirs)]
+    rows = -(-T // S) if integrate else T
+    out = api.DeviceArray.empty((rows, F, B), np.float32)
+    out.fill(0xFF)
+    dx, dpos, dfr, ddir = arrays
+    TR.multibeam_tracker_launch(None, dx, out, T, F, A, B, S, dpos, dfr, directions=ddir,
+                                integrate=integrate, kernel=kernel)
+    api.device_synchronize()
+    return out.to_numpy()
+
+
+@pytest.mark.parametrize("T,F,A,B,S,integrate,step", [
+    (1, 5, 64, 1, 10, True, 1e-3), (330, 17, 32, 9, 15, True, 1e-4),
+    (333, 336, 64, 17, 16, True, 1e-6), (700, 20, 64, 33, 17, True, 1e-2),
+    (500, 3, 128, 16, 10, True, 1e-2), (300, 3, 256, 9, 12, True, 1e-3),
+    (63, 9, 64, 8, 64, True, 1e-3), (191, 336, 32, 33, 64, True, 1e-3),
+    (400, 5, 64, 128, 100, True, 1e-3), (641, 336, 64, 31, 320, True, 1e-3),
+    (335, 2, 128, 24, 320, True, 1e-3), (335, 2, 256, 10, 320, True, 1e-3),
+    (100, 11, 64, 15, 10, False, 1e-4), (213, 7, 32, 20, 70, False, 1e-3),
+    (150, 5, 128, 17, 75, False, 1e-3), (90, 3, 256, 3, 80, False, 1e-3),
+])
+def test_sizes_vs_fp64(T, F, A, B, S, integrate, step):
+    x, pos, fr, dirs = case(T, F, A, B, S, T + A + B, step)
+    _, ref64 = O.multibeam_tracker(x, T, F, A, B, S, pos, fr, dirs, want_f64=True,
+                                   spectra=not integrate)
+    # a short last window holds less power than the floor of a whole one
+    floor = incoherent_floor(x, A, S if integrate else 1)
+    for kernel, tol in KERNELS:
+        got = launch(x, pos, fr, dirs, T, F, A, B, S, integrate, kernel)
+        assert rel_err_floored(got, ref64, floor) <= tol, kernel.name
+
+
+@pytest.mark.parametrize("S", [10, 64])
+def test_long_baselines_vs_fp64(S):
+    """3000 km: more turns than the integer form of the phase holds, next to
+    what it does hold; the FP64 phase itself is right to about 1e-9 turns."""
+    T, F, A, B = 130, 4, 64, 5
+    x, pos, fr, dirs = case(T, F, A, B, S, 3, step=1e-8, scale=1.0)
+    pos[::3] *= np.float32(4e5)
+    _, ref64 = O.multibeam_tracker(x, T, F, A, B, S, pos, fr, dirs, want_f64=True)
+    for kernel, tol in KERNELS:
+        got = launch(x, pos, fr, dirs, T, F, A, B, S, True, kernel)
+        assert rel_err_floored(got, ref64, incoherent_floor(x, A, S)) <= tol, kernel.name
+
+
+@pytest.mark.parametrize("S", [10, 64])
+def test_direction_that_is_not_a_number(S):
+    """A beam without a direction in some windows gives NaN there, and only
+    there: not for its other windows nor for other beams."""
+    T, F, A, B = 20 * S, 3, 64, 10
+    x, pos, fr, dirs = case(T, F, A, B, S, 9, step=1e-6)
+    want = launch(x, pos, fr, dirs, T, F, A, B, S, True, K.SPLIT_F16)
+    dirs[5:8, 3] = np.nan
+    dirs[17, 9, 2] = np.inf
+    got = launch(x, pos, fr, dirs, T, F, A, B, S, True, K.SPLIT_F16)
+    assert np.isnan(got[5:8, :, 3]).all() and np.isnan(got[17, :, 9]).all()
+    got[5:8, :, 3] = want[5:8, :, 3]
+    got[17, :, 9] = want[17, :, 9]
+    assert np.array_equal(got, want)
