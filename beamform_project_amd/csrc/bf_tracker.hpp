@@ -29,7 +29,8 @@ struct TrackerLaunch {
     Geom geo{};
     int dir_source = kDirTrajectory;
     const float* dir_table = nullptr;     // [n_windows][B][3]
-    const float* trajectories = nullptr;  // [B][4]
+    const float* trajectories = nullptr;  // [B][4], or null with one beam:
+    float trajectory[4] = {};             // its row by value
     size_t window_offset = 0;             // absolute index of window 0
     bool integrate = false;
     int kernel = BF_KERNEL_SPLIT_F16;

@@ -74,7 +74,6 @@ struct bf_opt_tracker {
     bool initialised = false;
     float start[3] = {0.0f, 0.0f, 1.0f};
     float rate[2] = {0.0f, 0.0f};
-    float h_traj[4] = {};     // staging of the trajectory row
     OptSearch h_search{};     // staging of the search state
     std::vector<float> h_dirs;  // [W][3] of the last run
     bool dirs_pending = false;  // h_dirs still on the device
@@ -104,7 +103,6 @@ struct bf_opt_tracker {
     OptSearch* d_search = nullptr;
     float* d_dirs = nullptr;
     size_t dirs_cap = 0;
-    float* d_traj = nullptr;
 
     ~bf_opt_tracker() {
         if (last_stream) (void)hipStreamSynchronize(last_stream);
@@ -114,7 +112,7 @@ struct bf_opt_tracker {
                             (void*)q.trace64, (void*)q.mode})
                 if (p) (void)hipFree(p);
         for (void* p : {(void*)d_pos, (void*)d_freqs, (void*)d_state, (void*)d_part,
-                        (void*)d_search, (void*)d_dirs, (void*)d_traj})
+                        (void*)d_search, (void*)d_dirs})
             if (p) (void)hipFree(p);
         for (hipEvent_t e : {ev_start, ev_ready[0], ev_ready[1], ev_used[0], ev_used[1], ev_done})
             if (e) (void)hipEventDestroy(e);
@@ -172,12 +170,8 @@ struct bf_opt_tracker {
         last_stream = stream;
         if (G <= 1) {
             const float traj[4] = {start[0], start[1], rate[0], rate[1]};
-            std::memcpy(h_traj, traj, sizeof(traj));
-            hip_check(hipMemcpyAsync(d_traj, h_traj, sizeof(h_traj), hipMemcpyHostToDevice,
-                                     stream),
-                      "hipMemcpyAsync trajectory");
+            std::memcpy(L_emit.trajectory, traj, sizeof(traj));
             L_emit.dir_source = kDirTrajectory;
-            L_emit.trajectories = d_traj;
             launch_tracker(stream, L_emit);
             hip_check(hipEventRecord(ev_done, stream), "hipEventRecord");
             ran = true;
@@ -327,7 +321,6 @@ void create_tracker(const float* positions, const float* frequencies, const bf_d
         hip_check(hipEventCreateWithFlags(e, hipEventDisableTiming), "hipEventCreate");
     t->d_part = dmalloc<float>(F * std::max<size_t>(t->G * t->G, 9));
     t->d_search = dmalloc<OptSearch>(1);
-    t->d_traj = dmalloc<float>(4);
     *out = std::move(t);
 }
 

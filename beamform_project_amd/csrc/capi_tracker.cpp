@@ -78,20 +78,9 @@ Geom default_geometry(size_t A) {
     return g;
 }
 
-// Per-beam trajectory row (l0, m0, rate_l, rate_m) passed by value through a
-// tiny device table owned by the caller's object or stream-ordered memory.
-struct TrajTable {
-    float v[4];
-};
-
-TrajTable traj_of(const bf_tracker_config& c) {
-    return TrajTable{{c.direction_start[0], c.direction_start[1],
-                      c.direction_rate_per_sample[0], c.direction_rate_per_sample[1]}};
-}
-
 TrackerLaunch single_beam_launch(const uint8_t* x, float* out, const bf_dims& d,
-                                 const bf_tracker_config& cfg, const float* d_traj,
-                                 size_t window_offset, int kernel) {
+                                 const bf_tracker_config& cfg, size_t window_offset,
+                                 int kernel) {
     TrackerLaunch L;
     L.x = x;
     L.out = out;
@@ -103,7 +92,11 @@ TrackerLaunch single_beam_launch(const uint8_t* x, float* out, const bf_dims& d,
     L.n_windows = ceil_div(d.n_time, cfg.integration_spectra);
     L.geo = default_geometry(d.n_ant);
     L.dir_source = kDirTrajectory;
-    L.trajectories = d_traj;
+    // (l0, m0, rate_l, rate_m) travels with the kernel's arguments
+    L.trajectory[0] = cfg.direction_start[0];
+    L.trajectory[1] = cfg.direction_start[1];
+    L.trajectory[2] = cfg.direction_rate_per_sample[0];
+    L.trajectory[3] = cfg.direction_rate_per_sample[1];
     L.window_offset = window_offset;
     L.integrate = false;
     L.kernel = kernel;
@@ -127,7 +120,6 @@ struct bf_tracker_stream {
     float last_ms = 0.0f;
     uint8_t* d_packed = nullptr;
     float* d_out = nullptr;
-    float* d_traj = nullptr;      // [1][4]
     size_t* d_offset = nullptr;   // unused placeholder kept zero
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
@@ -138,14 +130,13 @@ struct bf_tracker_stream {
         if (graph) (void)hipGraphDestroy(graph);
         if (d_packed) (void)hipFree(d_packed);
         if (d_out) (void)hipFree(d_out);
-        if (d_traj) (void)hipFree(d_traj);
         if (start) (void)hipEventDestroy(start);
         if (stop) (void)hipEventDestroy(stop);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
     void enqueue(size_t first_window) {
-        const TrackerLaunch L = single_beam_launch(d_packed, d_out, batch_dims, cfg, d_traj,
+        const TrackerLaunch L = single_beam_launch(d_packed, d_out, batch_dims, cfg,
                                                    first_window, kernel);
         launch_tracker(stream, L);
     }
@@ -195,16 +186,7 @@ bf_status bf_beam_tracker_device_resident(const uint8_t* d_packed, float* d_inte
             invalid("d_packed must be 16-byte aligned");
         const int kernel = tracker_kernel(exec);
         hipStream_t s = static_cast<hipStream_t>(stream);
-        // The trajectory row travels as a 16-byte kernel-visible table in
-        // stream-ordered memory (released on the same stream).
-        float* d_traj = nullptr;
-        hip_check(hipMallocAsync(reinterpret_cast<void**>(&d_traj), 16, s), "hipMallocAsync");
-        const TrajTable t = traj_of(*tracker);
-        hip_check(hipMemcpyAsync(d_traj, t.v, sizeof(t.v), hipMemcpyHostToDevice, s),
-                  "hipMemcpyAsync trajectory");
-        launch_tracker(s, single_beam_launch(d_packed, d_intensity, d, *tracker, d_traj, 0,
-                                             kernel));
-        hip_check(hipFreeAsync(d_traj, s), "hipFreeAsync");
+        launch_tracker(s, single_beam_launch(d_packed, d_intensity, d, *tracker, 0, kernel));
         if (stream == nullptr) hip_check(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
     });
 }
@@ -227,24 +209,18 @@ bf_status bf_beam_tracker_into(const uint8_t* packed, size_t packed_bytes, const
         hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate");
         uint8_t* dx = nullptr;
         float* dout = nullptr;
-        float* dtraj = nullptr;
         auto cleanup = [&] {
             if (dx) (void)hipFree(dx);
             if (dout) (void)hipFree(dout);
-            if (dtraj) (void)hipFree(dtraj);
             (void)hipStreamDestroy(s);
         };
         try {
             hip_check(hipMalloc(reinterpret_cast<void**>(&dx), n_in), "hipMalloc d_packed");
             hip_check(hipMalloc(reinterpret_cast<void**>(&dout), n_out * sizeof(float)),
                       "hipMalloc d_intensity");
-            hip_check(hipMalloc(reinterpret_cast<void**>(&dtraj), 16), "hipMalloc trajectory");
-            const TrajTable t = traj_of(*tracker);
-            hip_check(hipMemcpyAsync(dtraj, t.v, sizeof(t.v), hipMemcpyHostToDevice, s),
-                      "hipMemcpyAsync trajectory");
             hip_check(hipMemcpyAsync(dx, packed, n_in, hipMemcpyHostToDevice, s),
                       "hipMemcpyAsync H2D d_packed");
-            launch_tracker(s, single_beam_launch(dx, dout, d, *tracker, dtraj, 0, kernel));
+            launch_tracker(s, single_beam_launch(dx, dout, d, *tracker, 0, kernel));
             hip_check(hipMemcpyAsync(intensity, dout, n_out * sizeof(float),
                                      hipMemcpyDeviceToHost, s),
                       "hipMemcpyAsync D2H d_intensity");
@@ -285,10 +261,6 @@ bf_status bf_tracker_stream_create(const bf_dims* single_window_dims,
         hip_check(hipMalloc(reinterpret_cast<void**>(&s->d_out),
                             bd.n_time * bd.n_freq * sizeof(float)),
                   "hipMalloc d_intensity");
-        hip_check(hipMalloc(reinterpret_cast<void**>(&s->d_traj), 16), "hipMalloc trajectory");
-        const TrajTable t = traj_of(*tracker);
-        hip_check(hipMemcpy(s->d_traj, t.v, sizeof(t.v), hipMemcpyHostToDevice),
-                  "hipMemcpy trajectory");
         *out = s.release();
     });
 }

@@ -122,7 +122,7 @@ void serve_tasks_kernel(
         const int w_last = w_first + work->n_win[sidx];
         const int w_begin = w_first + rest / F * sl->wpi;
         const int w_end = w_begin + sl->wpi < w_last ? w_begin + sl->wpi : w_last;
-        const DirArgs da{nullptr, &sl->traj[0][0], 0L, sl->S, sl->B};
+        const DirArgs da{nullptr, &sl->traj[0][0], {}, 0L, sl->S, sl->B};
         const RowSource rs{ring + (size_t)f * A, (unsigned)(F * A), (long)ring_mask,
                            (long)sl->t0, (long)sl->t_end, MASKED ? valid + f : nullptr,
                            (size_t)F};
@@ -265,8 +265,11 @@ void launch_tracker(hipStream_t stream, const TrackerLaunch& L) {
         L.n_windows > (size_t)INT32_MAX / 2)
         fail(BF_ERR_OVERFLOW, "tracker grid exceeds the supported size");
     const bool table = L.dir_source == kDirTable;
+    const float* const q = L.trajectory;
     const DirArgs da{table ? L.dir_table : nullptr, table ? nullptr : L.trajectories,
-                     (long)L.window_offset, (int)L.S, (int)L.B};
+                     {q[0], q[1], q[2], q[3]}, (long)L.window_offset, (int)L.S, (int)L.B};
+    if (!table && L.trajectories == nullptr && L.B != 1)
+        invalid("a trajectory by value is for one beam");
     // One beam, per-spectrum output: the FP32 stream kernel (AUTO and FP32).
     if (L.B == 1 && !L.integrate &&
         (L.kernel == BF_KERNEL_AUTO || L.kernel == BF_KERNEL_FP32)) {

@@ -20,7 +20,8 @@ namespace bfhip {
 
 struct DirArgs {
     const float* table;  // directions [n_windows_table][B][3], or null for
-    const float* traj;   // trajectories [B][4] = l0, m0, rate_l, rate_m
+    const float* traj;   // trajectories [B][4] = l0, m0, rate_l, rate_m, or null for
+    float row[4];        // the only beam's trajectory
     long window_offset;  // absolute index of local window 0
     int S;
     int B;
@@ -36,7 +37,9 @@ __device__ __forceinline__ void beam_direction(const DirArgs& da, int w, int b, 
         d[1] = p[1];
         d[2] = p[2];
     } else {
-        const float* q = da.traj + (size_t)b * 4;
+        float q[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q[i] = da.traj != nullptr ? da.traj[(size_t)b * 4 + i] : da.row[i];
         const float tf = (float)((da.window_offset + w) * (long)da.S);
         const float l = q[0] + tf * q[2];
         const float m = q[1] + tf * q[3];
