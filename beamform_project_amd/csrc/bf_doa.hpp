@@ -15,6 +15,11 @@ size_t launch_doa_covariance(hipStream_t stream, const uint8_t* x, size_t T, siz
                              size_t A, size_t t0, size_t K, size_t M, int* rs, int* r_full,
                              size_t max_parts = 1);
 
+// The same for `n` consecutive windows of K snapshots from t0, the last one
+// cut short by T: rs [n][F][M][M][2], one part each.
+void launch_doa_covariance_windows(hipStream_t stream, const uint8_t* x, size_t T, size_t F,
+                                   size_t A, size_t t0, size_t K, size_t n, size_t M, int* rs);
+
 // FP64 fold, Cholesky, inverse and Bartlett/Capon scans per channel; rs
 // holds `parts` partial covariances, summed here.
 void launch_doa_fold_scan(hipStream_t stream, const int* rs, size_t parts, double* state,
@@ -46,29 +51,49 @@ struct OptGridArgs {
     int interp;    // quadratic peak interpolation
 };
 
-// Per channel: R_block = Rs / (K L) (forward-backward averaged when fb),
-// diagonal load (Capon), forgetting fold into state [F][M][M][2] FP64, and
-// the scan operand: Bartlett, the strict upper triangle of R in scanmat
-// [F][M][M] with its trace in trace[F] (mode 0); Capon, R^-1 in scan64
-// [F][M][M] with its trace in trace64[F] (mode 1), or the Bartlett form
-// where the factorisation fails.
-void launch_opt_fold(hipStream_t stream, const int* rs, double* state, bool first, size_t F,
-                     size_t M, size_t K, size_t L, bool fb, bool capon, float load,
-                     float lambda, float2* scanmat, float* trace, double2* scan64,
-                     double* trace64, int* mode);
+// Windows whose operands are prepared together at most.
+inline constexpr int kOptBatch = 4;
 
-// part[n_cells][F]: each channel's power at the cells of `level` (0: the
-// G x G grid around search->prev, else the 3 x 3 refinement candidates).
-void launch_opt_scan(hipStream_t stream, const float2* scanmat, const float* trace,
-                     const double2* scan64, const double* trace64, const int* mode,
-                     const float* pos, const float* freqs, const OptSearch* search,
-                     const OptGridArgs& g, int level, size_t F, size_t n_cells, bool capon,
-                     float* part);
+// Scan operands of `n` <= kOptBatch consecutive windows, per channel:
+// operand_bytes each, the trace, and the form (1: R^-1 in FP64; 0: R in
+// FP32).
+struct OptWindows {
+    size_t n = 0;
+    char* operand = nullptr;
+    double* trace = nullptr;
+    int* mode = nullptr;
+};
+size_t opt_operand_bytes(size_t M, bool capon);
+// Doubles of launch_opt_scan's scratch.
+size_t opt_part_count(size_t F, size_t n_cells);
 
-// Sums part over channels and takes the level's decision; at last_level
-// writes the window's direction to dirs[window][3].
-void launch_opt_decide(hipStream_t stream, const float* part, size_t F, size_t n_cells,
-                       const OptGridArgs& g, int level, int last_level, size_t window,
-                       OptSearch* search, float* dirs);
+// Per channel and window, in order: R_block = Rs / (K L) (forward-backward
+// averaged when fb; K_last snapshots in the last window), diagonal load
+// (Capon), forgetting fold into state [F][M][M][2] FP64, and the scan
+// operand: R, or Capon's R^-1, or R where its factorisation fails.
+void launch_opt_fold(hipStream_t stream, const OptWindows& b, const int* rs, double* state,
+                     bool first, size_t F, size_t M, size_t K, size_t K_last, size_t L, bool fb,
+                     bool capon, float load, float lambda);
+
+// The chain of scan launches of one run.  A launch reads state[n & 1], takes
+// the decision on launch n - 1 from part[(n - 1) & 1], leaves the new state in
+// state[(n + 1) & 1] and its own sums in part[n & 1].
+struct OptScan {
+    OptSearch* state = nullptr;          // [2]; state[0] set before the first launch
+    double* part[2] = {nullptr, nullptr};  // opt_part_count doubles each
+    unsigned launches = 0;               // of this run
+    int level = 0;                       // the last launch's
+    size_t cells = 0, groups = 0, window = 0;
+};
+
+// One level of the search of window `index` of the batch: every channel's
+// power at the cells (0: the G x G grid around the state's prev, else the 3 x
+// 3 refinement candidates), after the decision on the launch before, which
+// at last_level writes its window's direction to dirs[window][3].  With
+// n_cells = 0 only that decision is taken.
+void launch_opt_scan(hipStream_t stream, OptScan& q, const OptWindows& b, size_t index,
+                     const float* pos, const float* freqs, const OptGridArgs& g, int level,
+                     int last_level, size_t window, size_t F, size_t n_cells, bool capon,
+                     float* dirs);
 
 }  // namespace bfhip

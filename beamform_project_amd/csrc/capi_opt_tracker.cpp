@@ -16,6 +16,7 @@
 // launch over the whole shard with the estimated directions as its table.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -82,16 +83,11 @@ struct bf_opt_tracker {
     float* d_pos = nullptr;
     float* d_freqs = nullptr;
     double* d_state = nullptr;
-    // Per-window operands, two slots: the covariance, fold and factor of
-    // window w + 1 run on the prep stream while window w is searched.
-    struct Slot {
-        int* rs = nullptr;
-        float2* scan = nullptr;
-        float* trace = nullptr;
-        double2* scan64 = nullptr;  // Capon: R^-1 per channel
-        double* trace64 = nullptr;
-        int* mode = nullptr;
-    } slot[2];
+    // Scan operands of a batch of windows, two slots: the covariances, fold
+    // and factor of the next batch run on the prep stream while this one's
+    // windows are searched.
+    OptWindows slot[2];
+    int* d_rs = nullptr;  // [kOptBatch][F][M][M][2], of the batch in preparation
     hipStream_t prep = nullptr;
     // ev_done: the end of the last run on its stream; the next run's stream
     // (which may be another one) waits on it before it writes any state.
@@ -99,20 +95,19 @@ struct bf_opt_tracker {
     bool ran = false;
     hipEvent_t ev_start = nullptr, ev_ready[2] = {nullptr, nullptr},
                ev_used[2] = {nullptr, nullptr};
-    float* d_part = nullptr;
-    OptSearch* d_search = nullptr;
+    OptScan scan;
     float* d_dirs = nullptr;
     size_t dirs_cap = 0;
 
     ~bf_opt_tracker() {
         if (last_stream) (void)hipStreamSynchronize(last_stream);
         if (prep) (void)hipStreamSynchronize(prep);
-        for (const Slot& q : slot)
-            for (void* p : {(void*)q.rs, (void*)q.scan, (void*)q.trace, (void*)q.scan64,
-                            (void*)q.trace64, (void*)q.mode})
+        for (const OptWindows& q : slot)
+            for (void* p : {(void*)q.operand, (void*)q.trace, (void*)q.mode})
                 if (p) (void)hipFree(p);
-        for (void* p : {(void*)d_pos, (void*)d_freqs, (void*)d_state, (void*)d_part,
-                        (void*)d_search, (void*)d_dirs})
+        for (void* p : {(void*)d_rs, (void*)d_pos, (void*)d_freqs, (void*)d_state,
+                        (void*)scan.part[0], (void*)scan.part[1], (void*)scan.state,
+                        (void*)d_dirs})
             if (p) (void)hipFree(p);
         for (hipEvent_t e : {ev_start, ev_ready[0], ev_ready[1], ev_used[0], ev_used[1], ev_done})
             if (e) (void)hipEventDestroy(e);
@@ -182,7 +177,8 @@ struct bf_opt_tracker {
         }
         std::memcpy(h_search.prev, &prior[0], sizeof(h_search.prev));
         std::memcpy(h_search.centre, &prior[0], sizeof(h_search.centre));
-        hip_check(hipMemcpyAsync(d_search, &h_search, sizeof(h_search), hipMemcpyHostToDevice,
+        scan.launches = 0;
+        hip_check(hipMemcpyAsync(scan.state, &h_search, sizeof(h_search), hipMemcpyHostToDevice,
                                  stream),
                   "hipMemcpyAsync search");
         const OptGridArgs g = grid_args();
@@ -190,30 +186,35 @@ struct bf_opt_tracker {
         // The prep stream starts after the caller's prior work (the input).
         hip_check(hipEventRecord(ev_start, stream), "hipEventRecord");
         hip_check(hipStreamWaitEvent(prep, ev_start, 0), "hipStreamWaitEvent");
-        for (size_t w = 0; w < W; ++w) {
-            const int k = (int)(w & 1);
-            Slot& q = slot[k];
-            // prep: window w's operands into slot k, once window w - 2's
-            // search has released it
-            if (w >= 2) hip_check(hipStreamWaitEvent(prep, ev_used[k], 0), "hipStreamWaitEvent");
-            const size_t t0 = w * S;
-            const size_t K = std::min(S, T - t0);
-            launch_doa_covariance(prep, x, T, F, A, t0, K, M, q.rs, nullptr);
-            launch_opt_fold(prep, q.rs, d_state, !initialised, F, M, K, L, smoothing, capon,
-                            cfg.diagonal_load, cfg.forgetting_factor, q.scan, q.trace, q.scan64,
-                            q.trace64, q.mode);
+        // Batches of kOptBatch windows, after a first one of a single window,
+        // whose preparation nothing hides.
+        size_t begin = 0;
+        for (size_t batch = 0; begin < W; ++batch) {
+            const int k = (int)(batch & 1);
+            OptWindows& q = slot[k];
+            q.n = batch == 0 ? 1 : std::min<size_t>(kOptBatch, W - begin);
+            // prep: the batch's operands into slot k, once the search of the
+            // batch before the last has released it
+            if (batch >= 2)
+                hip_check(hipStreamWaitEvent(prep, ev_used[k], 0), "hipStreamWaitEvent");
+            const size_t t0 = begin * S;
+            const size_t K_last = std::min(S, T - (begin + q.n - 1) * S);
+            launch_doa_covariance_windows(prep, x, T, F, A, t0, S, q.n, M, d_rs);
+            launch_opt_fold(prep, q, d_rs, d_state, !initialised, F, M, S, K_last, L, smoothing,
+                            capon, cfg.diagonal_load, cfg.forgetting_factor);
             initialised = true;
             hip_check(hipEventRecord(ev_ready[k], prep), "hipEventRecord");
-            // search of window w on the caller's stream
+            // search of its windows on the caller's stream
             hip_check(hipStreamWaitEvent(stream, ev_ready[k], 0), "hipStreamWaitEvent");
-            for (int level = 0; level <= last; ++level) {
-                const size_t cells = level == 0 ? G * G : 9;
-                launch_opt_scan(stream, q.scan, q.trace, q.scan64, q.trace64, q.mode, d_pos,
-                                d_freqs, d_search, g, level, F, cells, capon, d_part);
-                launch_opt_decide(stream, d_part, F, cells, g, level, last, w, d_search, d_dirs);
-            }
+            for (size_t i = 0; i < q.n; ++i)
+                for (int level = 0; level <= last; ++level)
+                    launch_opt_scan(stream, scan, q, i, d_pos, d_freqs, g, level, last,
+                                    begin + i, F, level == 0 ? G * G : 9, capon, d_dirs);
             hip_check(hipEventRecord(ev_used[k], stream), "hipEventRecord");
+            begin += q.n;
         }
+        launch_opt_scan(stream, scan, slot[0], 0, d_pos, d_freqs, g, 0, last, W, F, 0, capon,
+                        d_dirs);  // the last decision
         L_emit.dir_source = kDirTable;
         L_emit.dir_table = d_dirs;
         launch_tracker(stream, L_emit);
@@ -304,23 +305,20 @@ void create_tracker(const float* positions, const float* frequencies, const bf_d
     hip_check(hipMemcpy(t->d_freqs, fr.data(), F * sizeof(float), hipMemcpyHostToDevice),
               "hipMemcpy frequencies");
     t->d_state = dmalloc<double>(F * M * M * 2);
-    for (auto& q : t->slot) {
-        q.rs = dmalloc<int>(F * M * M * 2);
-        q.scan = dmalloc<float2>(F * M * M);
-        q.trace = dmalloc<float>(F);
-        if (t->capon) {
-            q.scan64 = dmalloc<double2>(F * M * M);
-            q.trace64 = dmalloc<double>(F);
-        }
-        q.mode = dmalloc<int>(F);
+    for (OptWindows& q : t->slot) {
+        q.operand = dmalloc<char>(kOptBatch * F * opt_operand_bytes(M, t->capon));
+        q.trace = dmalloc<double>(kOptBatch * F);
+        q.mode = dmalloc<int>(kOptBatch * F);
     }
+    t->d_rs = dmalloc<int>(kOptBatch * F * M * M * 2);
     // default priority (a stream of another priority is never created here)
     hip_check(hipStreamCreateWithFlags(&t->prep, hipStreamNonBlocking), "hipStreamCreate");
     for (hipEvent_t* e : {&t->ev_done, &t->ev_start, &t->ev_ready[0], &t->ev_ready[1], &t->ev_used[0],
                           &t->ev_used[1]})
         hip_check(hipEventCreateWithFlags(e, hipEventDisableTiming), "hipEventCreate");
-    t->d_part = dmalloc<float>(F * std::max<size_t>(t->G * t->G, 9));
-    t->d_search = dmalloc<OptSearch>(1);
+    for (double*& p : t->scan.part)
+        p = dmalloc<double>(opt_part_count(F, std::max<size_t>(t->G * t->G, 9)));
+    t->scan.state = dmalloc<OptSearch>(2);
     *out = std::move(t);
 }
 

@@ -62,11 +62,13 @@ __device__ __forceinline__ void upper_tile(int t, int n, int* I, int* J) {
 // -> 2A components.  Part p (blockIdx.y) covers snapshots kpart p ..
 // kpart (p + 1) - 1 of the update (never empty: the launcher sizes the
 // parts) and writes its own smoothed partial sum to rs_out + p F M M 2;
-// the consumer adds the parts (integers, so in any order).  G is
+// the consumer adds the parts (integers, so in any order).  Window z
+// (blockIdx.z) covers the K snapshots from t0 + z K, as far as T goes, and
+// writes to rs_out + z F M M 2 (one part).  G is
 // symmetric, so only the tiles on and above the diagonal are accumulated;
 // every entry the covariance reads for r <= c lies there, and r > c is the
 // conjugate of (c, r).
-template <int A>
+template <int A, bool SMOOTH>
 __global__ __launch_bounds__(kThreads) void covariance_kernel(
     const uint8_t* __restrict__ x, int T, int F, int t0, int K, int M, int kpart,
     int* __restrict__ rs_out /* [parts][F][M][M][2] */,
@@ -76,7 +78,7 @@ __global__ __launch_bounds__(kThreads) void covariance_kernel(
     constexpr int TILES = NTILE * (NTILE + 1) / 2;  // upper triangle
     constexpr int PER_WAVE = (TILES + 3) / 4;
     __shared__ __attribute__((aligned(16))) unsigned char tr[C * kTStride];
-    __shared__ int g[C * (C + 1)];  // G, row stride C+1
+    __shared__ int g[SMOOTH ? C * (C + 1) : 1];  // G, row stride C+1
     // Workgroups are dealt round-robin to the 8 XCDs; give each XCD a
     // contiguous range of channels so that channels f and f+1, which share
     // the 128-byte lines of every packed row, meet in one L2.
@@ -85,9 +87,9 @@ __global__ __launch_bounds__(kThreads) void covariance_kernel(
     if (f >= F) return;  // whole workgroup
     {
         const int kb = (int)blockIdx.y * kpart;
-        t0 += kb;
-        K = min(K - kb, kpart);
-        rs_out += (size_t)blockIdx.y * F * M * M * 2;
+        t0 += (int)blockIdx.z * K + kb;
+        K = min(min(K - kb, kpart), T - t0);
+        rs_out += (size_t)(blockIdx.y + blockIdx.z) * F * M * M * 2;
     }
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -202,6 +204,30 @@ __global__ __launch_bounds__(kThreads) void covariance_kernel(
             take(kr + 64 * s, ring[s], cur);
             process(cur);
         }
+    }
+    if constexpr (!SMOOTH) {
+        // M = A: R straight from the accumulators.  A lane holds column l % 16
+        // (Re or Im of antenna b = l % 16 / 2) and both rows of the antennas
+        // 2 g and 2 g + 1 of its tile; with the partner's two rows the even
+        // lane forms R(2 g, b) and the odd one R(2 g + 1, b).
+        int2* rs2 = reinterpret_cast<int2*>(rs_out) + (size_t)f * A * A;
+        const bool odd = (lane & 1) != 0;
+#pragma unroll
+        for (int i = 0; i < PER_WAVE; ++i) {
+            if (wave * PER_WAVE + i >= TILES) break;
+            // mine: the two rows (re, im) of my antenna; theirs: of the other's
+            const int m0 = odd ? acc[i][2] : acc[i][0], m1 = odd ? acc[i][3] : acc[i][1];
+            const int o0 = odd ? acc[i][0] : acc[i][2], o1 = odd ? acc[i][1] : acc[i][3];
+            const int p0 = __shfl_xor(o0, 1), p1 = __shfl_xor(o1, 1);
+            const int a = 8 * tI[i] + 2 * (lane >> 4) + (odd ? 1 : 0);
+            const int b = 8 * tJ[i] + ((lane & 15) >> 1);
+            // even: columns (re: mine, im: partner's); odd: the reverse
+            const int re = (odd ? p0 + m1 : m0 + p1) / 256;
+            const int im = (odd ? p1 - m0 : m1 - p0) / 256;
+            rs2[a * A + b] = make_int2(re, im);
+            if (tI[i] != tJ[i]) rs2[b * A + a] = make_int2(re, -im);
+        }
+        return;
     }
     // G tiles -> LDS: lane holds column l%16, rows 4*(l/16) + r.
 #pragma unroll
@@ -610,7 +636,7 @@ size_t launch_doa_covariance(hipStream_t stream, const uint8_t* x, size_t T, siz
     const size_t kpart = 64 * ceil_div(ceil_div(K, 64), parts);
     const dim3 grid((unsigned)(8 * ceil_div(F, 8)), (unsigned)parts);
 #define BF_COV(A_)                                                                            \
-    hipLaunchKernelGGL(covariance_kernel<A_>, grid, dim3(kThreads), 0, stream, x, (int)T,    \
+    hipLaunchKernelGGL((covariance_kernel<A_, true>), grid, dim3(kThreads), 0, stream, x, (int)T,    \
                        (int)F, (int)t0, (int)K, (int)M, (int)kpart, rs, r_full)
     switch (A) {
     case 32: BF_COV(32); break;
@@ -620,6 +646,29 @@ size_t launch_doa_covariance(hipStream_t stream, const uint8_t* x, size_t T, siz
 #undef BF_COV
     hip_check(hipGetLastError(), "covariance_kernel launch");
     return parts;
+}
+
+void launch_doa_covariance_windows(hipStream_t stream, const uint8_t* x, size_t T, size_t F,
+                                   size_t A, size_t t0, size_t K, size_t n, size_t M, int* rs) {
+    if (K == 0 || n == 0 || t0 + (n - 1) * K >= T)
+        invalid("the covariance window exceeds the time axis");
+    const dim3 grid((unsigned)(8 * ceil_div(F, 8)), 1, (unsigned)n);
+    // without smoothing there is no G in LDS, which kept two workgroups to a CU
+#define BF_COV(A_, SMOOTH_)                                                                   \
+    hipLaunchKernelGGL((covariance_kernel<A_, SMOOTH_>), grid, dim3(kThreads), 0, stream, x,  \
+                       (int)T, (int)F, (int)t0, (int)K, (int)M, (int)K, rs, (int*)nullptr)
+    if (A == 32 && M == A)
+        BF_COV(32, false);
+    else if (A == 32)
+        BF_COV(32, true);
+    else if (A == 64 && M == A)
+        BF_COV(64, false);
+    else if (A == 64)
+        BF_COV(64, true);
+    else
+        invalid("the DOA covariance supports 32 or 64 antennas");
+#undef BF_COV
+    hip_check(hipGetLastError(), "covariance_kernel launch");
 }
 
 void launch_doa_fold_scan(hipStream_t stream, const int* rs, size_t parts, double* state,

@@ -2,26 +2,32 @@
 // searching path of the reference's CpuOptBeamTracker::run_into
 // (src/cpu_opt_beam_tracker.cpp:1619-2457), one integration window at a time.
 //
-// Per window (all stages stream-ordered, nothing returns to the host):
+// All stages are stream-ordered, nothing returns to the host.  For a batch of
+// windows at once:
 //   covariance      launch_doa_covariance (k_doa.hip): exact int32 sums of
-//                   x x^H over the window's snapshots, forward smoothing over
+//                   x x^H over each window's snapshots, forward smoothing over
 //                   L = A - M + 1 sub-arrays (:559-636).
 //   opt_fold        per channel, FP64: R_block = Rs / (K L), forward-backward
 //                   average when smoothing (:637-656, without the in-place
 //                   read of already-averaged entries), diagonal load for
 //                   Capon (:244-253, before the fold, :1803-1804), forgetting
-//                   fold R = lambda R + (1 - lambda) R_block (:1880-1892),
-//                   trace.
-//   opt_factor      Capon only, one wave per channel: Cholesky R = L L^H
-//                   (:398-421) and its inverse W = L^-1, so that
-//                   a^H R^-1 a = |W a|^2 (:423-437).
+//                   fold R = lambda R + (1 - lambda) R_block (:1880-1892)
+//                   window by window, trace.
+//   opt_factor      Capon only: R^-1 by Gauss-Jordan, whose pivots are those
+//                   of the Cholesky factorisation (:398-421).
+// Then per window and level, one launch:
 //   opt_scan        per (channel, cell): the steering vector
 //                   a_j = exp(-j k p_j . d) (:96-106) and the Bartlett power
 //                   tr(R) + 2 Re sum_{r<c} conj(a_r) R_rc a_c (:287-306) or
-//                   the Capon power 1 / |W a|^2.
-//   opt_decide      one workgroup: powers summed over channels, argmax, the
-//                   next level's centre, quadratic peak interpolation
-//                   (:830-853), and at the last level the window's direction.
+//                   the Capon power 1 / (a^H R^-1 a), on the matrix cores,
+//                   summed over a workgroup's channels.  Every workgroup of
+//                   the next launch first adds those sums up and takes the
+//                   level's decision for itself: argmax, the next centre,
+//                   quadratic peak interpolation (:830-853), and at the last
+//                   level the window's direction.  (A launch of its own for
+//                   the decision costs two more gaps per level; letting the
+//                   last workgroup decide costs each one a fence across the
+//                   XCDs, 105 us instead of 13 for 144 cells.)
 // Level 0 scans the G x G grid centred on the previous estimate
 // (build_centred_grid, :798-828); each refinement level scans the 3 x 3
 // neighbourhood of the running centre at half the previous pitch
@@ -39,11 +45,12 @@
 
 #include "bf_doa.hpp"
 #include "gauss_jordan.hpp"
+#include "steering.hpp"
 
 namespace bfhip {
 namespace {
 
-constexpr int kThreads = 256;
+constexpr int kFoldThreads = 512;
 
 struct cd {
     double re, im;
@@ -164,141 +171,15 @@ __device__ void clamp_direction(float l, float m, float out[3]) {
 }
 
 // ------------------------------------------------------------------ fold
-// One workgroup per channel, one covariance entry per thread and pass:
-// R_block = Rs / (K L), forward-backward averaged when fb (the mirrored
-// entry is read from Rs directly), diagonal load for Capon, and the fold
-// into state.  Bartlett also writes its scan operand and the trace of the
-// folded R; Capon's operand comes from opt_factor_kernel.
-__global__ __launch_bounds__(kThreads) void opt_fold_kernel(
-    const int* __restrict__ rs, double* __restrict__ state, int first, int M, int K, int L,
-    int fb, int capon, float load, float lambda, float2* __restrict__ scanmat,
-    float* __restrict__ trace_out, int* __restrict__ mode_out) {
-    __shared__ double s_diag[64];
-    __shared__ double s_eps;
-    const int f = blockIdx.x;
-    const int tid = threadIdx.x;
-    const int MM = M * M;
-    const double scale = 1.0 / ((double)K * (double)L);
-    const int* rf = rs + (size_t)f * MM * 2;
-    auto block = [&](int r, int c) -> cd {
-        const int e = r * M + c;
-        cd v{(double)rf[2 * e] * scale, (double)rf[2 * e + 1] * scale};
-        if (fb) {
-            // (R + J conj(R) J) / 2
-            const int m = (M - 1 - r) * M + (M - 1 - c);
-            v.re = 0.5 * (v.re + (double)rf[2 * m] * scale);
-            v.im = 0.5 * (v.im - (double)rf[2 * m + 1] * scale);
-        }
-        return v;
-    };
-    if (tid < M) s_diag[tid] = block(tid, tid).re;
-    __syncthreads();
-    if (tid == 0) {
-        double tr = 0.0;
-        for (int i = 0; i < M; ++i) tr += s_diag[i];
-        s_eps = (capon && load > 0.0f) ? (double)load * tr / (double)M : 0.0;
-    }
-    __syncthreads();
-    const double eps = s_eps;
-    const double lam = (double)lambda;
-    const double comp = (double)(1.0f - lambda);
-    const bool copy = first || lambda >= 1.0f;
-    double* st = state + (size_t)f * MM * 2;
-    float2* Q = scanmat + (size_t)f * MM;
-    for (int e = tid; e < MM; e += kThreads) {
-        const int r = e / M, c = e - (e / M) * M;
-        cd v = block(r, c);
-        if (r == c) v.re += eps;
-        if (!copy) {
-            v.re = lam * st[2 * e] + comp * v.re;
-            v.im = lam * st[2 * e + 1] + comp * v.im;
-        }
-        st[2 * e] = v.re;
-        st[2 * e + 1] = v.im;
-        if (r == c) s_diag[r] = v.re;
-        // Bartlett operand: the strict upper triangle, zero elsewhere.
-        if (!capon)
-            Q[e] = r < c ? make_float2((float)v.re, (float)v.im) : make_float2(0.0f, 0.0f);
-    }
-    if (capon) return;
-    __syncthreads();
-    if (tid == 0) {
-        double tr = 0.0;
-        for (int i = 0; i < M; ++i) tr += s_diag[i];
-        trace_out[f] = (float)tr;
-        mode_out[f] = 0;
-    }
-}
-
-// ---------------------------------------------------------------- factor
-constexpr int kGjBlock = 4;                                     // 4 x 4 blocks
-constexpr int kFactorThreads = (64 / kGjBlock) * (64 / kGjBlock);  // 256
-// Capon operand: Q = R^-1 of the folded state by in-place Gauss-Jordan
-// elimination in FP64, one workgroup per channel.  Thread t holds the 4 x 4
-// block (rows 4 (t / 16) .., columns 4 (t % 16) ..) of a 64 x 64 matrix in
-// registers (identity beyond M); per pivot k the owners publish row k and
-// column k to LDS (double-buffered: one barrier per pivot) and every thread
-// updates its block.  Without pivoting on a Hermitian positive-definite R
-// the k-th pivot is the Cholesky pivot d_k = L_kk^2, so the reference's
-// factorisation test (d_k > 1e-12, :398-421) is applied to it; a failed
-// channel falls back to the Bartlett form on the folded R (:354-375).
-// Q is written in full (FP64) with its trace; the scan evaluates
-// 1 / (tr Q + 2 Re sum_{r<c} conj(a_r) Q_rc a_c) = 1 / (a^H R^-1 a) in
-// FP64, where the large entries of R^-1 cancel.
-__global__ __launch_bounds__(kFactorThreads) void opt_factor_kernel(
-    const double* __restrict__ state, int M, double2* __restrict__ scan64,
-    double* __restrict__ trace64, float2* __restrict__ scanmat, float* __restrict__ trace_out,
-    int* __restrict__ mode_out) {
-    __shared__ GjShared<cd> sh;
-    __shared__ double s_diag[64];
-    const int f = blockIdx.x;
-    const int tid = threadIdx.x;
-    const int i0 = gj_row0<kGjBlock>(tid), j0 = gj_col0<kGjBlock>(tid);
-    const int MM = M * M;
-    const double* R = state + (size_t)f * MM * 2;
-    cd a[kGjBlock][kGjBlock];
-    gj_load<kGjBlock>(a, R, M, M, tid);
-    const bool ok = gj_invert<kGjBlock>(a, M, 1e-12, sh, tid);
-    if (!ok) {
-        float2* Q = scanmat + (size_t)f * MM;
-        for (int e = tid; e < MM; e += kFactorThreads) {
-            const int r = e / M, c = e - (e / M) * M;
-            Q[e] = r < c ? make_float2((float)R[2 * e], (float)R[2 * e + 1])
-                         : make_float2(0.0f, 0.0f);
-        }
-        if (tid == 0) {
-            double tr = 0.0;
-            for (int i = 0; i < M; ++i) tr += R[2 * (i * M + i)];
-            trace_out[f] = (float)tr;
-            mode_out[f] = 0;
-        }
-        return;
-    }
-    double2* Q = scan64 + (size_t)f * MM;
-#pragma unroll
-    for (int u = 0; u < kGjBlock; ++u)
-#pragma unroll
-        for (int v = 0; v < kGjBlock; ++v) {
-            const int i = i0 + u, j = j0 + v;
-            if (i < M && j < M) {
-                Q[i * M + j] = make_double2(a[u][v].re, a[u][v].im);
-                if (i == j) s_diag[i] = a[u][v].re;
-            }
-        }
-    __syncthreads();
-    if (tid == 0) {
-        double tr = 0.0;
-        for (int i = 0; i < M; ++i) tr += s_diag[i];
-        trace64[f] = tr;
-        mode_out[f] = 1;
-    }
-}
-
-// ------------------------------------------------------------------ scan
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+// The scan's operand of one channel: the Hermitian form H = X + iY (R, or
+// R^-1) without its diagonal, which the trace carries, as two real planes
+// [Mp][Mp], Mp = M rounded up to 16, zero outside M.  Only the 16 x 16 blocks
+// (I, J) with J >= I are read; a block on the diagonal is read whole, so its
+// X is halved (exactly): the scan doubles every sum.  FP64 planes keep the
+// columns of a block in the order c -> 4 (c % 4) + c / 4, so that a lane's
+// four values of a block row are contiguous in both precisions.
+__device__ __forceinline__ int plane_column64(int c) {
+    return (c & ~15) | (4 * (c & 3) + ((c & 15) >> 2));
 }
 
 __device__ __forceinline__ double wave_sum_f64(double v) {
@@ -307,231 +188,303 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
     return v;
 }
 
-// One pass of a wave over NC cells: acc_lane = sum_r conj(a_r) R[r][lane]
-// over the strict upper triangle of R, a_r broadcast from this wave's LDS
-// steering vectors.  R is a zero-padded 64 x 64 tile and a_r = 0 for
-// r >= M, so rows are taken four at a time (the four LDS reads issue
-// together) up to M rounded up.
-template <int NC>
-__device__ __forceinline__ void scan_pass(const float2* __restrict__ Q,
-                                          const float2* __restrict__ sa, int M, int lane,
-                                          float2 (&acc)[NC]) {
-    for (int r0 = 0; r0 < M; r0 += 4) {
-        float2 q[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) q[u] = Q[(r0 + u) * 64 + lane];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int r = r0 + u;
-#pragma unroll
-            for (int j = 0; j < NC; ++j) {
-                const float2 av = sa[j * 64 + r];  // broadcast
-                const float ar = av.x, ai = av.y;
-                acc[j].x = fmaf(ai, q[u].y, fmaf(ar, q[u].x, acc[j].x));
-                acc[j].y = fmaf(-ai, q[u].x, fmaf(ar, q[u].y, acc[j].y));
-            }
-        }
-    }
-}
+// The windows of one batch, in order.
+struct FoldArgs {
+    const int2* rs;  // [n][F][M][M]
+    double2* state;  // [F][M][M]
+    char* operand;   // [n][F] operands of operand_bytes
+    double* trace;   // [n][F]
+    int* mode;       // [n][F]
+    size_t operand_bytes;
+    int n, first, M, Mp, K, K_last, L, fb, capon;
+    float load, lambda;
+};
 
-// Bartlett form: P = tr(R) + 2 Re sum_c y_c a_c (also Capon's fallback).
-template <int NC>
-__device__ void scan_cells(const float2* __restrict__ Q, float2* __restrict__ sa,
-                           const OptSearch& s,
-                           const OptGridArgs& g, int level, int c_begin, int c_end, int lane,
-                           int wave, int f, int F, double kw, float tr, float px, float py,
-                           float pz, float* __restrict__ part) {
-    const bool live = lane < g.M;
-    for (int c0 = c_begin + wave * NC; c0 < c_end; c0 += 4 * NC) {
-        float2 a[NC], acc[NC];
-#pragma unroll
-        for (int j = 0; j < NC; ++j) {
-            a[j] = make_float2(0.0f, 0.0f);
-            acc[j] = make_float2(0.0f, 0.0f);
-            const int cell = min(c0 + j, c_end - 1);
-            float dir[3];
-            double st[3];
-            cell_direction(g, s, level, cell, dir, st);
-            if (live) {
-                const double ph = kw * ((double)px * st[0] + (double)py * st[1] + (double)pz * st[2]);
-                double sn, cs;
-                sincos(ph, &sn, &cs);
-                a[j] = make_float2((float)cs, -(float)sn);
-            }
-            sa[j * 64 + lane] = a[j];
-        }
-        // the wave's own LDS writes precede its reads in order
-        __builtin_amdgcn_wave_barrier();
-        scan_pass<NC>(Q, sa, g.M, lane, acc);
-#pragma unroll
-        for (int j = 0; j < NC; ++j) {
-            float t = acc[j].x * a[j].x - acc[j].y * a[j].y;  // Re(y_c a_c)
-            t = wave_sum(t);
-            float p = tr + 2.0f * t;
-            if (!isfinite(p)) p = 0.0f;
-            if (lane == 0 && c0 + j < c_end) part[(size_t)(c0 + j) * F + f] = p;
-        }
-    }
-}
-
-// Capon in FP64: P = 1 / (tr Q + 2 Re sum_{r<c} conj(a_r) Q_rc a_c) with
-// Q = R^-1 (strict upper triangle in Q64, zero-padded to 64 x 64).
-template <int NC>
-__device__ void scan_cells_capon64(const double2* __restrict__ Q64, double2* __restrict__ sa,
-                                   const OptSearch& s,
-                                   const OptGridArgs& g, int level, int c_begin, int c_end,
-                                   int lane, int wave, int f, int F, double kw, double tr,
-                                   float px, float py, float pz, float* __restrict__ part) {
-    const bool live = lane < g.M;
-    for (int c0 = c_begin + wave * NC; c0 < c_end; c0 += 4 * NC) {
-        double2 a[NC], acc[NC];
-#pragma unroll
-        for (int j = 0; j < NC; ++j) {
-            a[j] = make_double2(0.0, 0.0);
-            acc[j] = make_double2(0.0, 0.0);
-            const int cell = min(c0 + j, c_end - 1);
-            float dir[3];
-            double st[3];
-            cell_direction(g, s, level, cell, dir, st);
-            if (live) {
-                const double ph = kw * ((double)px * st[0] + (double)py * st[1] + (double)pz * st[2]);
-                double sn, cs;
-                sincos(ph, &sn, &cs);
-                a[j] = make_double2(cs, -sn);
-            }
-            sa[j * 64 + lane] = a[j];
-        }
-        __builtin_amdgcn_wave_barrier();
-        for (int r0 = 0; r0 < g.M; r0 += 4) {
-            double2 q[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) q[u] = Q64[(r0 + u) * 64 + lane];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int r = r0 + u;
-#pragma unroll
-                for (int j = 0; j < NC; ++j) {
-                    const double2 av = sa[j * 64 + r];  // broadcast
-                    const double ar = av.x, ai = av.y;
-                    acc[j].x = fma(ai, q[u].y, fma(ar, q[u].x, acc[j].x));
-                    acc[j].y = fma(-ai, q[u].x, fma(ar, q[u].y, acc[j].y));
-                }
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < NC; ++j) {
-            double t = acc[j].x * a[j].x - acc[j].y * a[j].y;
-            t = wave_sum_f64(t);
-            const double den = tr + 2.0 * t;
-            float p = den > 1.0e-12 ? (float)(1.0 / den) : 0.0f;
-            if (!isfinite(p)) p = 0.0f;
-            if (lane == 0 && c0 + j < c_end) part[(size_t)(c0 + j) * F + f] = p;
-        }
-    }
-}
-
-// grid (F, chunks); part[cell][f] = the channel's power at the cell.
-template <int NC, int NC64>
-__global__ __launch_bounds__(kThreads) void opt_scan_kernel(
-    const float2* __restrict__ scanmat, const float* __restrict__ trace,
-    const double2* __restrict__ scan64, const double* __restrict__ trace64,
-    const int* __restrict__ mode, const float* __restrict__ pos, const float* __restrict__ freqs,
-    const OptSearch* __restrict__ search, OptGridArgs g, int level, int n_cells,
-    int cells_per_chunk, int F, int capon_run, float* __restrict__ part) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    float2* Q = reinterpret_cast<float2*>(smem);
-    double2* Q64 = reinterpret_cast<double2*>(smem);
+// One workgroup per channel: each thread carries its covariance entries
+// through the batch's windows: R_block = Rs / (K L), forward-backward averaged
+// when fb (the mirrored entry is read from Rs directly), diagonal load for
+// Capon, and the fold.  Bartlett writes the scan's FP32 planes, for the
+// entries of the blocks that are read; Capon the folded R, [M][M] complex FP64
+// in the operand's place, for opt_factor_kernel.  Bound by memory latency: an
+// entry's loads of all windows are issued together.
+__global__ __launch_bounds__(kFoldThreads) void opt_fold_kernel(FoldArgs a) {
+    __shared__ double s_eps[kOptBatch];
     const int f = blockIdx.x;
-    const bool capon64 = mode[f] == 1;
-    // per-wave steering vectors [NC][64] after the operand tile
-    unsigned char* steer = smem + 64 * 64 * (capon_run ? sizeof(double2) : sizeof(float2));
-    const int M = g.M;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int c_begin = (int)blockIdx.y * cells_per_chunk;
-    const int c_end = min(n_cells, c_begin + cells_per_chunk);
-    if (capon64) {
-        // strict upper triangle of R^-1, zero elsewhere
-        const double2* src = scan64 + (size_t)f * M * M;
-        for (int e = tid; e < 64 * 64; e += kThreads) {
-            const int r = e >> 6, c = e & 63;
-            Q64[e] = (r < c && c < M) ? src[r * M + c] : make_double2(0.0, 0.0);
-        }
-    } else {
-        // [64][64], zero outside [M][M] (M may be odd: element by element)
-        const float2* src = scanmat + (size_t)f * M * M;
-        for (int e = tid; e < 64 * 64; e += kThreads) {
-            const int r = e >> 6, c = e & 63;
-            Q[e] = (r < M && c < M) ? src[r * M + c] : make_float2(0.0f, 0.0f);
-        }
-    }
-    __syncthreads();
-    const OptSearch s = *search;
-    const float tr = trace[f];
-    const double kw = kTwoPi * (double)freqs[f] / kSpeedOfLight;
-    float px = 0.0f, py = 0.0f, pz = 0.0f;
-    if (lane < M) {
-        px = pos[3 * lane];
-        py = pos[3 * lane + 1];
-        pz = pos[3 * lane + 2];
-    }
-    if (capon64)
-        scan_cells_capon64<NC64>(Q64, reinterpret_cast<double2*>(steer) + wave * NC64 * 64, s,
-                                 g, level, c_begin, c_end, lane, wave, f, F, kw, trace64[f],
-                           px, py, pz, part);
-    else
-        scan_cells<NC>(Q, reinterpret_cast<float2*>(steer) + wave * NC * 64, s, g,
-                             level, c_begin, c_end, lane, wave, f, F, kw, tr, px, py, pz,
-                         part);
-}
-
-// ---------------------------------------------------------------- decide
-constexpr int kDecideThreads = 1024;
-
-// One workgroup: each wave sums a cell's channel powers (FP64, a fixed
-// lane-strided order and shuffle tree), then thread 0 takes the level's
-// serial decision.
-__global__ __launch_bounds__(kDecideThreads) void opt_decide_kernel(
-    const float* __restrict__ part, int F, int n_cells, OptGridArgs g, int level,
-    int last_level, int window, OptSearch* __restrict__ search, float* __restrict__ dirs) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    float* P = reinterpret_cast<float*>(smem);
+    const int F = gridDim.x;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
-    // four cells per wave at a time and kSteps channel steps of 64 per
-    // round: every load of a round is issued (at a clamped, in-bounds
-    // address) before the sums, which add in the order f = lane, lane + 64,
-    // ... as one loop over f would
-    constexpr int kWaves = kDecideThreads / 64;
-    constexpr int kSteps = 6;
-    for (int c0 = wave; c0 < n_cells; c0 += 4 * kWaves) {
-        double sum[4] = {0.0, 0.0, 0.0, 0.0};
-        for (int f0 = lane; f0 < F; f0 += 64 * kSteps) {
-            float v[kSteps][4];
+    const int M = a.M, MM = M * M;
+    const bool copy_all = a.lambda >= 1.0f;
+    const double lam = (double)a.lambda;
+    const double comp = (double)(1.0f - a.lambda);
+    // R_block of entry (r, c) in every window of the batch
+    auto blocks = [&](int r, int c, cd (&v)[kOptBatch]) {
+        int2 p[kOptBatch], m[kOptBatch];
 #pragma unroll
-            for (int k = 0; k < kSteps; ++k)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int f = min(f0 + 64 * k, F - 1);
-                    const int cell = min(c0 + j * kWaves, n_cells - 1);
-                    v[k][j] = part[(size_t)cell * F + f];
-                }
-#pragma unroll
-            for (int k = 0; k < kSteps; ++k)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (f0 + 64 * k < F && c0 + j * kWaves < n_cells) sum[j] += (double)v[k][j];
+        for (int w = 0; w < kOptBatch; ++w) {
+            const int2* rf = a.rs + ((size_t)min(w, a.n - 1) * F + f) * MM;
+            p[w] = rf[r * M + c];
+            if (a.fb) m[w] = rf[(M - 1 - r) * M + (M - 1 - c)];
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const double v = wave_sum_f64(sum[j]);
-            const int cell = c0 + j * kWaves;
-            if (lane == 0 && cell < n_cells) P[cell] = (float)v;
+        for (int w = 0; w < kOptBatch; ++w) {
+            const double scale = 1.0 / ((double)(w + 1 == a.n ? a.K_last : a.K) * (double)a.L);
+            v[w] = cd{(double)p[w].x * scale, (double)p[w].y * scale};
+            if (a.fb) {
+                // (R + J conj(R) J) / 2
+                v[w].re = 0.5 * (v[w].re + (double)m[w].x * scale);
+                v[w].im = 0.5 * (v[w].im - (double)m[w].y * scale);
+            }
+        }
+    };
+    double2* st = a.state + (size_t)f * MM;
+    if (wave == 0) {  // traces (M <= 64: one lane per diagonal entry)
+        cd v[kOptBatch];
+        const int i = min(lane, M - 1);
+        blocks(i, i, v);
+        // of the folded R, by the recursion below on the diagonal
+        double d = a.first || copy_all ? 0.0 : st[i * M + i].x;
+#pragma unroll
+        for (int w = 0; w < kOptBatch; ++w) {
+            if (w >= a.n) break;
+            const double tr = wave_sum_f64(lane < M ? v[w].re : 0.0);
+            d = copy_all || (a.first && w == 0) ? v[w].re : lam * d + comp * v[w].re;
+            const double folded = wave_sum_f64(lane < M ? d : 0.0);
+            if (lane == 0) {
+                s_eps[w] = (a.capon && a.load > 0.0f) ? (double)a.load * tr / (double)M : 0.0;
+                if (!a.capon) {
+                    a.trace[(size_t)w * F + f] = folded;
+                    a.mode[(size_t)w * F + f] = 0;
+                }
+            }
         }
     }
+    __syncthreads();  // and the diagonal's old state has been read
+    const int Mp = a.Mp;
+    // thread = column c of rows r0, r0 + step, ...
+    const int c = tid & 63, step = kFoldThreads / 64;
+    if (c >= Mp) return;
+    for (int r = tid >> 6; r < Mp; r += step) {
+        if (!a.capon && (r >> 4) > (c >> 4)) continue;
+        const bool in = r < M && c < M;
+        const int es = in ? r * M + c : 0;
+        cd v[kOptBatch];
+        blocks(min(r, M - 1), min(c, M - 1), v);
+        const double2 old = a.first || copy_all ? make_double2(0.0, 0.0) : st[es];
+        cd prev{old.x, old.y};
+#pragma unroll
+        for (int w = 0; w < kOptBatch; ++w) {
+            if (w >= a.n) break;
+            if (r == c) v[w].re += s_eps[w];
+            if (!copy_all && !(a.first && w == 0)) {
+                v[w].re = lam * prev.re + comp * v[w].re;
+                v[w].im = lam * prev.im + comp * v[w].im;
+            }
+            prev = v[w];
+            char* const op = a.operand + ((size_t)w * F + f) * a.operand_bytes;
+            if (a.capon) {
+                if (in) reinterpret_cast<double2*>(op)[es] = make_double2(prev.re, prev.im);
+            } else {
+                float* const X = reinterpret_cast<float*>(op) + r * Mp + c;
+                const bool zero = !in || r == c;
+                X[0] = zero ? 0.0f : ((r >> 4) == (c >> 4) ? 0.5f : 1.0f) * (float)prev.re;
+                X[Mp * Mp] = zero ? 0.0f : (float)prev.im;
+            }
+        }
+        if (in) st[es] = make_double2(prev.re, prev.im);
+    }
+}
+
+// ---------------------------------------------------------------- factor
+constexpr int kGjBlock = 4;                                     // 4 x 4 blocks
+constexpr int kFactorThreads = (64 / kGjBlock) * (64 / kGjBlock);  // 256
+// Capon operand: Q = R^-1 of the folded covariance by in-place Gauss-Jordan
+// elimination in FP64 (gauss_jordan.hpp), one workgroup per (channel,
+// window).  The reference's factorisation test (d_k > 1e-12, :398-421) is
+// applied to the pivots; a failed channel falls back to the Bartlett form on
+// the folded R (:354-375).  Bound by the chain of M pivots, each a barrier
+// and an FP64 division: a batch of windows in one launch keeps several
+// workgroups per CU in flight (10 windows of 64 antennas, 336 channels: 1.48
+// ms one window at a time).
+__global__ __launch_bounds__(kFactorThreads) void opt_factor_kernel(
+    char* __restrict__ operand, size_t operand_bytes, int M, int Mp, double* __restrict__ trace,
+    int* __restrict__ mode) {
+    __shared__ GjShared<cd> sh;
+    __shared__ double s_diag[64];
+    const size_t f = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
+    const int tid = threadIdx.x;
+    const int i0 = gj_row0<kGjBlock>(tid), j0 = gj_col0<kGjBlock>(tid);
+    char* const op = operand + f * operand_bytes;
+    const double* R = reinterpret_cast<const double*>(op);
+    cd a[kGjBlock][kGjBlock];
+    gj_load<kGjBlock>(a, R, M, M, tid);
+    const bool ok = gj_invert<kGjBlock>(a, M, 1e-12, sh, tid);
+    if (!ok) gj_load<kGjBlock>(a, R, M, M, tid);  // R again, in place
+    __syncthreads();  // R has been read by all before the planes replace it
+#pragma unroll
+    for (int u = 0; u < kGjBlock; ++u)
+#pragma unroll
+        for (int v = 0; v < kGjBlock; ++v) {
+            const int i = i0 + u, j = j0 + v;
+            if (i >= Mp || j >= Mp) continue;
+            const bool in = i < M && j < M && i != j;
+            const double half = (i >> 4) == (j >> 4) ? 0.5 : 1.0;
+            const double re = in ? half * a[u][v].re : 0.0, im = in ? a[u][v].im : 0.0;
+            if (ok) {
+                double* const X = reinterpret_cast<double*>(op);
+                X[i * Mp + plane_column64(j)] = re;
+                X[(Mp + i) * Mp + plane_column64(j)] = im;
+            } else {
+                float* const X = reinterpret_cast<float*>(op);
+                X[i * Mp + j] = (float)re;
+                X[(Mp + i) * Mp + j] = (float)im;
+            }
+            if (i == j) s_diag[i] = i < M ? a[u][v].re : 0.0;
+        }
     __syncthreads();
-    if (wave != 0) return;
+    if (tid < 64) {
+        const double tr = wave_sum_f64(tid < M ? s_diag[tid] : 0.0);
+        if (tid == 0) {
+            trace[f] = tr;
+            mode[f] = ok ? 1 : 0;
+        }
+    }
+}
+
+// ------------------------------------------------------------------ scan
+// With a = u + iv and H = X + iY (X symmetric, Y antisymmetric, both without
+// the diagonal), a^H H a = tr H + 2 sum_{r<c} Re(conj(a_r) H_rc a_c).  By 16 x
+// 16 blocks that is 2 sum_I [u_I . (U - Z) + v_I . (V + W)] with U, V =
+// sum_{J >= I} X_IJ u_J, X_IJ v_J, W = sum_{J >= I} Y_IJ u_J and Z =
+// sum_{J > I} Y_IJ v_J (a diagonal block needs no Z: v . Y u counts both of its
+// triangles).  A wave evaluates 16 cells of one channel, a column each:
+// the four sums are 16x16x4 MFMAs (FP32, or FP64 for Capon, where the large
+// entries of R^-1 cancel), with H's rows as the A operand straight from L2.
+// Lane l holds cell l % 16 and a quarter of the antennas (g = l / 16):
+// slot 4 J + r is antenna 16 J + 4 g + r in FP32 and 16 J + 4 r + g in FP64, the
+// rows its MFMA results hold, so u, v meet U, V, W, Z without moving.
+typedef double bf_double4 __attribute__((ext_vector_type(4)));
+
+template <typename T>
+struct ScanTypes;
+template <>
+struct ScanTypes<float> {
+    typedef bf_float4 vec;
+    __device__ static vec mfma(float a, float b, vec c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    __device__ static int antenna(int j, int r, int g) { return 16 * j + 4 * g + r; }
+};
+template <>
+struct ScanTypes<double> {
+    typedef bf_double4 vec;
+    __device__ static vec mfma(double a, double b, vec c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    __device__ static int antenna(int j, int r, int g) { return 16 * j + 4 * r + g; }
+};
+
+// This lane's part of sum_I [...] over the block rows I = i0, i1 (i1 < 0: all
+// rows from i0) of the cell whose phase per metre (in turns) is d.
+template <typename T>
+__device__ __forceinline__ T scan_form(const T* __restrict__ X, int Mp, const double* s_pos,
+                                       const double (&d)[3], unsigned rows, int lane) {
+    using ST = ScanTypes<T>;
+    typedef typename ST::vec vec;
+    const int g = lane >> 4;
+    const int nb = Mp >> 4;
+    T u[16], v[16];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const double* const p = s_pos + 3 * ST::antenna(j, r, g);
+            const double t = fma(p[2], d[2], fma(p[1], d[1], p[0] * d[0]));
+            const double2 cs = cos_sin_turns64(t);
+            u[4 * j + r] = (T)cs.x;
+            v[4 * j + r] = (T)-cs.y;
+        }
+    const T* const row = X + (size_t)(lane & 15) * Mp + 4 * g;  // + 16 I Mp + 16 J
+    T sum = (T)0;
+#pragma unroll
+    for (int I = 0; I < 4; ++I) {
+        if (I >= nb || !((rows >> I) & 1u)) continue;  // uniform
+        vec U = {0, 0, 0, 0}, V = {0, 0, 0, 0}, W = {0, 0, 0, 0}, Z = {0, 0, 0, 0};
+#pragma unroll
+        for (int J = I; J < 4; ++J) {
+            if (J >= nb) continue;
+            const vec x = *reinterpret_cast<const vec*>(row + (size_t)16 * I * Mp + 16 * J);
+            const vec y = *reinterpret_cast<const vec*>(row + (size_t)(Mp + 16 * I) * Mp + 16 * J);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                U = ST::mfma(x[r], u[4 * J + r], U);
+                V = ST::mfma(x[r], v[4 * J + r], V);
+                W = ST::mfma(y[r], u[4 * J + r], W);
+                if (J > I) Z = ST::mfma(y[r], v[4 * J + r], Z);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            sum += u[4 * I + r] * (U[r] - Z[r]) + v[4 * I + r] * (V[r] + W[r]);
+    }
+    return sum;
+}
+
+struct ScanArgs {
+    const char* operand;  // the window's [F] operands
+    const double* trace;  // [F]
+    const int* mode;      // [F]
+    size_t operand_bytes;
+    const float* pos;
+    const float* freqs;
+    const OptSearch* search;  // the state before that launch's decision
+    OptGridArgs g;
+    int level, n_cells, F, Mp;
+    double* part;  // [groups][16 tiles] sums over the channels of a workgroup
+    // the launch before this one, whose decision is taken here
+    int last_level, before_level, before_cells, before_groups, before_window;
+    const double* before_part;  // null: no launch before
+    OptSearch* next;  // the state after that decision
+    float* dirs;
+};
+
+constexpr int kScanWaves = 8;
+constexpr int kScanThreads = 64 * kScanWaves;
+
+// The decision on the launch before, by the whole workgroup: its powers summed
+// over the channel groups, in FP64 and a fixed order (`ways` threads per cell,
+// their partial sums in LDS), then thread 0's serial part; the new state goes
+// to *out.  P and sums: LDS scratch.
+__device__ void decide(const ScanArgs& a, float* P, double* sums, OptSearch* out) {
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int n_cells = a.before_cells;
+    const int padded = (n_cells + 15) & ~15;
+    const int level = a.before_level, last_level = a.last_level;
+    const OptGridArgs& g = a.g;
+    const int ways = padded < kScanThreads ? kScanThreads / padded : 1;
+    const int per = (a.before_groups + ways - 1) / ways;
+    for (int i = tid; i < padded * ways; i += kScanThreads) {
+        const int cell = i % padded, way = i / padded;
+        const int end = min(a.before_groups, (way + 1) * per);
+        double sum = 0.0;
+#pragma unroll 8
+        for (int q = way * per; q < end; ++q) sum += a.before_part[(size_t)q * padded + cell];
+        if (ways > 1)
+            sums[i] = sum;
+        else
+            P[cell] = (float)sum;
+    }
+    __syncthreads();
+    if (ways > 1) {
+        for (int cell = tid; cell < n_cells; cell += kScanThreads) {
+            double sum = 0.0;
+            for (int way = 0; way < ways; ++way) sum += sums[way * padded + cell];
+            P[cell] = (float)sum;
+        }
+        __syncthreads();
+    }
+    if (tid >= 64) return;
     // argmax with the reference's rule (strict >, so the first maximum):
     // each lane scans its cells in increasing order, then the lanes combine
     // preferring the larger value and, on a tie, the lower index
@@ -552,10 +505,10 @@ __global__ __launch_bounds__(kDecideThreads) void opt_decide_kernel(
         }
     }
     if (lane != 0) return;
-    OptSearch s = *search;
-    const int best = bi;
+    OptSearch s = *a.search;
     float dir[3];
     double st[3];
+    const int best = bi;
     cell_direction(g, s, level, best, dir, st);
     float c[3] = {dir[0], dir[1], dir[2]};
     if (g.interp) {
@@ -588,71 +541,172 @@ __global__ __launch_bounds__(kDecideThreads) void opt_decide_kernel(
         s.prev[0] = c[0];
         s.prev[1] = c[1];
         s.prev[2] = c[2];
-        dirs[3 * window] = c[0];
-        dirs[3 * window + 1] = c[1];
-        dirs[3 * window + 2] = c[2];
+        if (blockIdx.x == 0 && blockIdx.y == 0)
+            for (int i = 0; i < 3; ++i) a.dirs[3 * a.before_window + i] = c[i];
     }
-    *search = s;
+    *out = s;
+    if (blockIdx.x == 0 && blockIdx.y == 0) *a.next = s;
+}
+
+// Grid (channel groups, tiles of 16 cells).  A workgroup's eight waves take
+// eight channels; with HALVES (the nine refinement cells, where the time of
+// one wave is what counts) four, and each wave two of the four block rows:
+// {0, 3} or {1, 2}, 72 MFMAs either way.  A launch without cells only takes the
+// decision on the one before.
+template <bool CAPON, bool HALVES>
+__global__ __launch_bounds__(kScanThreads) void opt_scan_kernel(ScanArgs a) {
+    constexpr int kChannels = HALVES ? kScanWaves / 2 : kScanWaves;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    __shared__ double s_sums[kScanThreads];
+    __shared__ double s_pos[3 * 64];
+    __shared__ double s_form[kScanWaves][16];
+    __shared__ OptSearch s_search;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int f0 = blockIdx.x * kChannels;
+    const int f = f0 + (HALVES ? wave >> 1 : wave);
+    for (int i = tid; i < 3 * 64; i += kScanThreads)
+        s_pos[i] = i < 3 * a.g.M ? (double)a.pos[i] : 0.0;
+    if (a.before_part != nullptr) {
+        decide(a, reinterpret_cast<float*>(smem), s_sums, &s_search);
+    } else if (tid == 0) {
+        s_search = *a.search;
+        if (blockIdx.x == 0 && blockIdx.y == 0) *a.next = s_search;
+    }
+    __syncthreads();
+    if (a.n_cells == 0) return;
+    float dir[3];
+    double st[3];
+    const int cell = min((int)blockIdx.y * 16 + (lane & 15), a.n_cells - 1);
+    cell_direction(a.g, s_search, a.level, cell, dir, st);
+    if (f < a.F) {
+        const double per_metre = turns_per_metre(a.freqs[f]);
+        const double d[3] = {st[0] * per_metre, st[1] * per_metre, st[2] * per_metre};
+        const char* const op = a.operand + (size_t)f * a.operand_bytes;
+        const unsigned rows = HALVES ? ((wave & 1) ? 0x6u : 0x9u) : 0xFu;
+        double form;
+        if (CAPON && a.mode[f] == 1)
+            form = scan_form<double>(reinterpret_cast<const double*>(op), a.Mp, s_pos, d, rows,
+                                     lane);
+        else
+            form = (double)scan_form<float>(reinterpret_cast<const float*>(op), a.Mp, s_pos, d,
+                                            rows, lane);
+        form += __shfl_xor(form, 16);
+        form += __shfl_xor(form, 32);
+        if (lane < 16) s_form[wave][lane] = form;
+    }
+    __syncthreads();
+    if (tid < 16) {
+        double sum = 0.0;
+        for (int i = 0; i < kChannels && f0 + i < a.F; ++i) {
+            const double form = HALVES ? s_form[2 * i][tid] + s_form[2 * i + 1][tid]
+                                       : s_form[i][tid];
+            const double q = a.trace[f0 + i] + 2.0 * form;
+            float p;
+            if (CAPON && a.mode[f0 + i] == 1)
+                p = q > 1.0e-12 ? (float)(1.0 / q) : 0.0f;
+            else
+                p = (float)q;
+            if (!isfinite(p)) p = 0.0f;
+            sum += (double)p;
+        }
+        a.part[((size_t)blockIdx.x * gridDim.y + blockIdx.y) * 16 + tid] = sum;
+    }
 }
 
 }  // namespace
 
-void launch_opt_fold(hipStream_t stream, const int* rs, double* state, bool first, size_t F,
-                     size_t M, size_t K, size_t L, bool fb, bool capon, float load,
-                     float lambda, float2* scanmat, float* trace, double2* scan64,
-                     double* trace64, int* mode) {
-    hipLaunchKernelGGL(opt_fold_kernel, dim3((unsigned)F), dim3(kThreads), 0, stream, rs, state,
-                       first ? 1 : 0, (int)M, (int)K, (int)L, fb ? 1 : 0, capon ? 1 : 0, load,
-                       lambda, scanmat, trace, mode);
+size_t opt_operand_bytes(size_t M, bool capon) {
+    const size_t Mp = 16 * ceil_div(M, 16);
+    return 2 * Mp * Mp * (capon ? sizeof(double) : sizeof(float));
+}
+
+size_t opt_part_count(size_t F, size_t n_cells) {
+    return 16 * ceil_div(n_cells, 16) * ceil_div(F, kScanWaves / 2);
+}
+
+void launch_opt_fold(hipStream_t stream, const OptWindows& b, const int* rs, double* state,
+                     bool first, size_t F, size_t M, size_t K, size_t K_last, size_t L, bool fb,
+                     bool capon, float load, float lambda) {
+    FoldArgs a{};
+    a.rs = reinterpret_cast<const int2*>(rs);
+    a.state = reinterpret_cast<double2*>(state);
+    a.operand = b.operand;
+    a.trace = b.trace;
+    a.mode = b.mode;
+    a.operand_bytes = opt_operand_bytes(M, capon);
+    a.n = (int)b.n;
+    a.first = first ? 1 : 0;
+    a.M = (int)M;
+    a.Mp = 16 * (int)ceil_div(M, 16);
+    a.K = (int)K;
+    a.K_last = (int)K_last;
+    a.L = (int)L;
+    a.fb = fb ? 1 : 0;
+    a.capon = capon ? 1 : 0;
+    a.load = load;
+    a.lambda = lambda;
+    hipLaunchKernelGGL(opt_fold_kernel, dim3((unsigned)F), dim3(kFoldThreads), 0, stream, a);
     hip_check(hipGetLastError(), "opt_fold_kernel launch");
     if (!capon) return;
-    hipLaunchKernelGGL(opt_factor_kernel, dim3((unsigned)F), dim3(kFactorThreads), 0, stream, state,
-                       (int)M, scan64, trace64, scanmat, trace, mode);
+    hipLaunchKernelGGL(opt_factor_kernel, dim3((unsigned)F, (unsigned)b.n), dim3(kFactorThreads),
+                       0, stream, b.operand, a.operand_bytes, a.M, a.Mp, b.trace, b.mode);
     hip_check(hipGetLastError(), "opt_factor_kernel launch");
 }
 
-void launch_opt_scan(hipStream_t stream, const float2* scanmat, const float* trace,
-                     const double2* scan64, const double* trace64, const int* mode,
-                     const float* pos, const float* freqs, const OptSearch* search,
-                     const OptGridArgs& g, int level, size_t F, size_t n_cells, bool capon,
-                     float* part) {
-    // One pass per wave: cells are spread over as many workgroups as it
-    // takes (each stages its channel's operand once), which keeps the
-    // per-wave chain short; the 3 x 3 refinement uses three waves of 3.
-    const bool coarse = level == 0;
-    const size_t per_wave = coarse ? (capon ? 4 : 8) : 3;
-    const size_t cpc = 4 * per_wave;
-    const size_t chunks = ceil_div(n_cells, cpc);
-    // operand tile, then per-wave steering vectors (sized for either path)
-    const size_t nc = coarse ? 8 : 3, nc64 = coarse ? 4 : 3;  // the template arguments
-    const size_t steer_per_wave =
-        64 * std::max(nc * sizeof(float2), capon ? nc64 * sizeof(double2) : 0);
-    const size_t smem = 64 * 64 * (capon ? sizeof(double2) : sizeof(float2)) + 4 * steer_per_wave;
-    const void* fn = coarse ? reinterpret_cast<const void*>(opt_scan_kernel<8, 4>)
-                            : reinterpret_cast<const void*>(opt_scan_kernel<3, 3>);
-    if (smem > 64 * 1024)
-        hip_check(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem),
-                  "hipFuncSetAttribute");
-#define BF_OPT_SCAN(NC_, NC64_)                                                                \
-    hipLaunchKernelGGL((opt_scan_kernel<NC_, NC64_>), dim3((unsigned)F, (unsigned)chunks),      \
-                       dim3(kThreads), smem, stream, scanmat, trace, scan64, trace64, mode, pos,  \
-                       freqs, search, g, level, (int)n_cells, (int)cpc, (int)F, capon ? 1 : 0,  \
-                       part)
-    if (coarse)
-        BF_OPT_SCAN(8, 4);
+void launch_opt_scan(hipStream_t stream, OptScan& q, const OptWindows& b, size_t index,
+                     const float* pos, const float* freqs, const OptGridArgs& g, int level,
+                     int last_level, size_t window, size_t F, size_t n_cells, bool capon,
+                     float* dirs) {
+    ScanArgs a{};
+    a.operand_bytes = opt_operand_bytes((size_t)g.M, capon);
+    a.operand = b.operand + index * F * a.operand_bytes;
+    a.trace = b.trace + index * F;
+    a.mode = b.mode + index * F;
+    a.pos = pos;
+    a.freqs = freqs;
+    a.g = g;
+    a.level = level;
+    a.n_cells = (int)n_cells;
+    a.F = (int)F;
+    a.Mp = 16 * (int)ceil_div((size_t)g.M, 16);
+    a.last_level = last_level;
+    const unsigned now = q.launches & 1u;
+    a.part = q.part[now];
+    a.search = q.state + now;
+    a.next = q.state + (now ^ 1u);
+    a.dirs = dirs;
+    if (q.launches > 0) {
+        a.before_part = q.part[now ^ 1u];
+        a.before_level = q.level;
+        a.before_cells = (int)q.cells;
+        a.before_groups = (int)q.groups;
+        a.before_window = (int)q.window;
+    }
+    // one tile cannot fill the chip: half the work per wave
+    const size_t tiles = ceil_div(n_cells, 16);
+    const bool halves = tiles <= 1;
+    const size_t groups = n_cells == 0 ? 1 : ceil_div(F, halves ? kScanWaves / 2 : kScanWaves);
+    const dim3 grid((unsigned)groups, (unsigned)std::max<size_t>(tiles, 1));
+    const size_t smem = std::max<size_t>(q.cells, 1) * sizeof(float);
+#define BF_SCAN(C_, H_) \
+    hipLaunchKernelGGL((opt_scan_kernel<C_, H_>), grid, dim3(kScanThreads), smem, stream, a)
+    if (capon && halves)
+        BF_SCAN(true, true);
+    else if (capon)
+        BF_SCAN(true, false);
+    else if (halves)
+        BF_SCAN(false, true);
     else
-        BF_OPT_SCAN(3, 3);
-#undef BF_OPT_SCAN
+        BF_SCAN(false, false);
+#undef BF_SCAN
     hip_check(hipGetLastError(), "opt_scan_kernel launch");
-}
-
-void launch_opt_decide(hipStream_t stream, const float* part, size_t F, size_t n_cells,
-                       const OptGridArgs& g, int level, int last_level, size_t window,
-                       OptSearch* search, float* dirs) {
-    hipLaunchKernelGGL(opt_decide_kernel, dim3(1), dim3(kDecideThreads), n_cells * sizeof(float),
-                       stream,
-                       part, (int)F, (int)n_cells, g, level, last_level, (int)window, search, dirs);
-    hip_check(hipGetLastError(), "opt_decide_kernel launch");
+    ++q.launches;
+    q.level = level;
+    q.cells = n_cells;
+    q.groups = groups;
+    q.window = window;
 }
 
 }  // namespace bfhip

@@ -98,6 +98,38 @@ __device__ __forceinline__ float2 cos_sin_turns(unsigned i) {
     return make_float2(__builtin_bit_cast(float, cs), __builtin_bit_cast(float, sn));
 }
 
+// cos and sin of v turns in FP64, any finite v (else NaN): the quadrant split
+// off exactly, then the Taylor series on |x| <= pi/4 (to x^17 and x^16: the
+// next terms are below 2^-56).
+__device__ __forceinline__ double2 cos_sin_turns64(double v) {
+    const double v4 = 4.0 * (v - rint(v));  // exact
+    const double n = rint(v4);
+    const double x = (v4 - n) * (0.25 * kTwoPi);
+    const double z = x * x;
+    double p = 1.0 / 355687428096000.0;
+    p = fma(z, p, -1.0 / 1307674368000.0);
+    p = fma(z, p, 1.0 / 6227020800.0);
+    p = fma(z, p, -1.0 / 39916800.0);
+    p = fma(z, p, 1.0 / 362880.0);
+    p = fma(z, p, -1.0 / 5040.0);
+    p = fma(z, p, 1.0 / 120.0);
+    p = fma(z, p, -1.0 / 6.0);
+    double q = 1.0 / 20922789888000.0;
+    q = fma(z, q, -1.0 / 87178291200.0);
+    q = fma(z, q, 1.0 / 479001600.0);
+    q = fma(z, q, -1.0 / 3628800.0);
+    q = fma(z, q, 1.0 / 40320.0);
+    q = fma(z, q, -1.0 / 720.0);
+    q = fma(z, q, 1.0 / 24.0);
+    q = fma(z, q, -0.5);
+    const double s = fma(x * z, p, x);
+    const double c = fma(z, q, 1.0);
+    const int quad = (int)n & 3;  // n = -2 .. 2
+    const double cs = (quad & 1) ? s : c;
+    const double sn = (quad & 1) ? c : s;
+    return make_double2((quad == 1 || quad == 2) ? -cs : cs, (quad & 2) ? -sn : sn);
+}
+
 // Turns per metre of a channel.
 __device__ __forceinline__ double turns_per_metre(float f_hz) {
     return (double)f_hz / kSpeedOfLight;
