@@ -168,7 +168,7 @@ __global__ __launch_bounds__(kB1WavesPerBlock * 64) void beam1_stream_kernel(
     const int t0 = min(tw0 + c * per, tw1);
     const int t1 = min(t0 + per, tw1);
     float d[3];
-    beam_direction(da, w, 0, d);
+    beam_direction(da, beam_row(da, 0), w, 0, d);
     float reach[3];
     geometry_reach<A>(geo, lane, reach);
     const Steer st = make_steer(d, turns_per_metre(channel_frequency(geo, fl)), reach);

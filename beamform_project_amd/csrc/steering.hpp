@@ -27,19 +27,32 @@ struct DirArgs {
     int B;
 };
 
+// What a beam's direction is made of besides the window: its trajectory's row
+// (kept in registers over a run of windows), or nothing with a table.
+struct BeamRow {
+    float q[4];
+};
+__device__ __forceinline__ BeamRow beam_row(const DirArgs& da, int b) {
+    BeamRow r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        r.q[i] = da.table != nullptr ? 0.0f
+                                     : (da.traj != nullptr ? da.traj[(size_t)b * 4 + i] : da.row[i]);
+    return r;
+}
+
 // Direction of beam b in local window w: the table's, or
 // l = l0 + (float)t * rate_l, n = sqrt(1 - l^2 - m^2)
 // (src/beam_tracker.cpp:166-179, src/geometry.cpp:97-106).
-__device__ __forceinline__ void beam_direction(const DirArgs& da, int w, int b, float d[3]) {
+__device__ __forceinline__ void beam_direction(const DirArgs& da, const BeamRow& row, int w, int b,
+                                               float d[3]) {
     if (da.table != nullptr) {
         const float* p = da.table + ((size_t)w * da.B + b) * 3;
         d[0] = p[0];
         d[1] = p[1];
         d[2] = p[2];
     } else {
-        float q[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) q[i] = da.traj != nullptr ? da.traj[(size_t)b * 4 + i] : da.row[i];
+        const float* q = row.q;
         const float tf = (float)((da.window_offset + w) * (long)da.S);
         const float l = q[0] + tf * q[2];
         const float m = q[1] + tf * q[3];

@@ -203,9 +203,9 @@ struct Channel {
 // even lane evaluates j = 0, 2 and the odd lane j = 1, 3; each slices its own
 // and takes the partner's by DPP.
 template <int A, int NT, int PARTS, bool ANCHORED>
-__device__ __forceinline__ void window_operands(const DirArgs& da, const Channel<A>& ch, int w,
-                                                int beam0, int lane, bool direct,
-                                                WeightAnchor<A, NT>& anc,
+__device__ __forceinline__ void window_operands(const DirArgs& da, const BeamRow (&rows)[NT],
+                                                const Channel<A>& ch, int w, int beam0, int lane,
+                                                bool direct, WeightAnchor<A, NT>& anc,
                                                 bf_uint4v (&bw)[PARTS][NT][A / 16]) {
     constexpr int KS = A / 16;
     const int c = lane & 15;
@@ -215,79 +215,97 @@ __device__ __forceinline__ void window_operands(const DirArgs& da, const Channel
     const int a0 = g * (A / 4) + (odd ? 1 : 0);  // own antennas a0 + 4 s + 2 jj
     const bool anchored = ANCHORED && !direct;
     const int wa = w - w % kAnchorWindows;
-    // This lane's two weights of k-step s; `near`: every lane's phases fit the
-    // integer form (wave-uniform).  Columns past the last beam hold the
+    // Direction of column c's beam.  Columns past the last beam hold the
     // weights of direction 0; they are not stored.
-    auto own_weights = [&](const Steer& st, bool near, int s, float2 (&v)[2]) {
-        const double* const p = ch.pos.d + 3 * (a0 + 4 * s);
-        if (__builtin_expect(near, 1)) {
-            v[0] = steering_weight_near(p, st);
-            v[1] = steering_weight_near(p + 6, st);
-        } else {
-            v[0] = steering_weight_any(p, st);
-            v[1] = steering_weight_any(p + 6, st);
-        }
+    auto direction = [&](int nt, int window, float (&d)[3]) {
+        const int b = beam0 + nt * 8 + (c >> 1);
+        d[0] = d[1] = d[2] = 0.0f;
+        if (b < da.B) beam_direction(da, rows[nt], window, b, d);
     };
     if (anchored && anc.window != wa) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            const int b = beam0 + nt * 8 + (c >> 1);
-            float d[3] = {0.0f, 0.0f, 0.0f};
-            if (b < da.B) beam_direction(da, wa, b, d);
+            float d[3];
+            direction(nt, wa, d);
 #pragma unroll
             for (int i = 0; i < 3; ++i) anc.dir[nt][i] = d[i];
             const Steer st = make_steer(d, ch.per_metre, ch.reach);
+            auto fill = [&](auto weight) {
 #pragma unroll
-            for (int s = 0; s < KS; ++s) own_weights(st, __all(st.in_range), s, anc.own[nt][s]);
+                for (int s = 0; s < KS; ++s)
+#pragma unroll
+                    for (int jj = 0; jj < 2; ++jj)
+                        anc.own[nt][s][jj] = weight(ch.pos.d + 3 * (a0 + 4 * s + 2 * jj), st);
+            };
+            if (__all(st.in_range))
+                fill(steering_weight_near);
+            else
+                fill(steering_weight_any);
         }
         anc.window = wa;
     }
     const float kf = (float)(kTwoPi * ch.per_metre);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-        const int b = beam0 + nt * 8 + (c >> 1);
-        float d[3] = {0.0f, 0.0f, 0.0f};
-        if (b < da.B) beam_direction(da, w, b, d);
-        const Steer st = make_steer(d, ch.per_metre, ch.reach);
+        float d[3];
+        direction(nt, w, d);
         float dk[3] = {0.0f, 0.0f, 0.0f};
         bool rotate = anchored;  // this lane's beam, from its anchor
-        if (anchored && w != wa) {
+        if (anchored) {
             float bound = 0.0f;
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
+                // (0 at the anchor itself: the rotation leaves it as it is)
                 dk[i] = kf * (d[i] - anc.dir[nt][i]);
                 bound += ch.reach[i] * fabsf(dk[i]);
             }
-            rotate = bound < 0.125f;
+            rotate = bound < 0.125f || (w == wa);
+            if (w == wa) dk[0] = dk[1] = dk[2] = 0.0f;
         }
-        const bool none_evaluate = __all(rotate);
-        const bool near = __all(st.in_range);
+        // k-steps one after another, each with its weights from `make`; only
+        // LDS reads may move across, which hides their latency (13 beams,
+        // windows of 10, 64 antennas: 232 -> 201 us); at 256 antennas there
+        // are no registers for that
+        auto steps = [&](auto make) {
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            float2 v[2];
-            if (!ANCHORED || !none_evaluate) own_weights(st, near, s, v);
-            if (ANCHORED && rotate) {
+            for (int s = 0; s < KS; ++s) {
+                float2 v[2];
 #pragma unroll
-                for (int jj = 0; jj < 2; ++jj) {
-                    // (by 0 at the anchor itself, which leaves it as it is)
-                    const float* p = ch.pos.s + 3 * (a0 + 4 * s + 2 * jj);
-                    const float t = fmaf(p[2], dk[2], fmaf(p[1], dk[1], p[0] * dk[0]));
-                    v[jj] = rotate_phasor(anc.own[nt][s][jj], t);
+                for (int jj = 0; jj < 2; ++jj) v[jj] = make(s, jj);
+                unsigned re[PARTS], im[PARTS];
+                slice_pair<PARTS>(v[0].x, v[1].x, re);
+                slice_pair<PARTS>(v[0].y, v[1].y, im);
+#pragma unroll
+                for (int q = 0; q < PARTS; ++q) {
+                    // (read by all lanes, outside the selects)
+                    const unsigned er = dpp_even(re[q]), ei = dpp_even(im[q]);
+                    const unsigned pr = dpp_odd(re[q]), pi = dpp_odd(im[q]);
+                    bw[q][nt][s] = bf_uint4v{odd ? ei : re[q], odd ? er : im[q] ^ flip,
+                                             odd ? im[q] : pr, (odd ? re[q] : pi) ^ flip};
                 }
+                __builtin_amdgcn_sched_barrier(A <= 128 ? 0x100 : 0);
             }
-            unsigned re[PARTS], im[PARTS];
-            slice_pair<PARTS>(v[0].x, v[1].x, re);
-            slice_pair<PARTS>(v[0].y, v[1].y, im);
-#pragma unroll
-            for (int q = 0; q < PARTS; ++q) {
-                // (read by all lanes, outside the selects)
-                const unsigned er = dpp_even(re[q]), ei = dpp_even(im[q]);
-                const unsigned pr = dpp_odd(re[q]), pi = dpp_odd(im[q]);
-                bw[q][nt][s] = bf_uint4v{odd ? ei : re[q], odd ? er : im[q] ^ flip,
-                                         odd ? im[q] : pr, (odd ? re[q] : pi) ^ flip};
-            }
-            // keeps the next step's loads and sums out of this one (registers)
-            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto rotated = [&](int s, int jj) {
+            const float* p = ch.pos.s + 3 * (a0 + 4 * s + 2 * jj);
+            const float t = fmaf(p[2], dk[2], fmaf(p[1], dk[1], p[0] * dk[0]));
+            return rotate_phasor(anc.own[nt][s][jj], t);
+        };
+        if (ANCHORED && __all(rotate)) {
+            steps(rotated);
+            continue;
+        }
+        const Steer st = make_steer(d, ch.per_metre, ch.reach);
+        if (!anchored && __all(st.in_range)) {
+            steps([&](int s, int jj) {
+                return steering_weight_near(ch.pos.d + 3 * (a0 + 4 * s + 2 * jj), st);
+            });
+        } else {
+            steps([&](int s, int jj) {
+                float2 v = steering_weight_any(ch.pos.d + 3 * (a0 + 4 * s + 2 * jj), st);
+                if (ANCHORED && rotate) v = rotated(s, jj);
+                return v;
+            });
         }
     }
 }
@@ -372,6 +390,9 @@ __device__ __forceinline__ void wave_windows(const RowSource& rs, const Channel<
 
     bf_uint4v bw[PARTS][NT][KS];
     WeightAnchor<A, NT> anc;
+    BeamRow rows[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) rows[nt] = beam_row(da, min(bl + 8 * nt, B - 1));
 #pragma unroll 1
     for (int w = w_begin; w < w_end; ++w) {
         const long t_win = rs.t_base + (long)w * S;
@@ -459,7 +480,7 @@ __device__ __forceinline__ void wave_windows(const RowSource& rs, const Channel<
             for (int u = 0; u < D; ++u)
                 if (u < tpw) buf[u] = load_tile(u);
         }
-        window_operands<A, NT, PARTS, ANCHORED>(da, ch, w, beam0, lane, direct, anc, bw);
+        window_operands<A, NT, PARTS, ANCHORED>(da, rows, ch, w, beam0, lane, direct, anc, bw);
         if (n_fast > 0) {
             bf_uint4v av[2][KS];
             auto group = [&](auto more, int j0) {
@@ -533,8 +554,15 @@ __device__ __forceinline__ void wave_windows(const RowSource& rs, const Channel<
     }
 }
 
+// Two waves per SIMD, or three where they almost fit by themselves (one
+// N-tile, few antennas: windows of 10, 320 spectra, 64 antennas 16 against 19 us).
+constexpr int min_waves(int A, int NT, int PARTS) {
+    return NT == 1 && A <= 64 && PARTS <= 2 ? 3 : 2;
+}
+
 template <int A, int NT, int PARTS, bool INTEGRATE, bool ANCHORED>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(min_waves(A, NT, PARTS))))
 void tracker_wave_kernel(const uint8_t* __restrict__ x, Geom geo, DirArgs da,
                          float* __restrict__ out, int T, int F, int n_windows, int run, int blocks,
                          long n_tasks, int per_xcd) {
