@@ -17,10 +17,14 @@
 
 namespace bfhip {
 
+// Row k's entry j = BS bj + v sits at v NB + bj (columns alike), so that the
+// blocks' reads of one v are contiguous: at BS bj + v sixteen of them share
+// four bank groups.
 template <typename Cd>
 struct GjShared {
     Cd row[2][64];
     Cd col[2][64];
+    double recip[2];
 };
 
 // Loads the block of a row-major M x M matrix with row stride ld (re, im at
@@ -49,67 +53,71 @@ __device__ __forceinline__ void gj_load(Cd (&a)[BS][BS], const double* src, int 
 
 // Inverts in place (M <= NB BS, which the caller guarantees); returns false
 // (uniformly) at the first pivot k < M that is not above `floor`, leaving
-// the block unspecified.
+// the block unspecified.  Pivots run block row by block row, so that every
+// register index is static and a pivot's owners are found by one comparison;
+// each thread divides for the next pivot along with its updates (only the
+// owner's quotient is published), which takes the FP64 division out of the
+// chain between barriers.
 template <int BS, int NB = 64 / BS, typename Cd>
 __device__ bool gj_invert(Cd (&a)[BS][BS], int M, double floor, GjShared<Cd>& sh, int tid) {
     static_assert(NB * BS <= 64, "the published row and column hold 64 entries");
-    const int i0 = gj_row0<BS, NB>(tid), j0 = gj_col0<BS, NB>(tid);
+    const int bi = tid / NB, bj = tid % NB;
+    double recip = 1.0 / a[0][0].re;
     // pivots beyond M act on the identity padding only: skipped
-    for (int k = 0; k < M; ++k) {
-        const int buf = k & 1;
-        // static register indices only (a runtime index would spill a[][])
+#pragma unroll 1
+    for (int kb = 0; kb < NB; ++kb) {
+        const bool in_row = bi == kb, in_col = bj == kb;
 #pragma unroll
-        for (int u = 0; u < BS; ++u)
-            if (i0 + u == k) {
+        for (int ku = 0; ku < BS; ++ku) {
+            const int k = kb * BS + ku;
+            if (k >= M) return true;  // uniform
+            const int buf = k & 1;
+            if (in_row) {
 #pragma unroll
-                for (int v = 0; v < BS; ++v) sh.row[buf][j0 + v] = a[u][v];
+                for (int v = 0; v < BS; ++v) sh.row[buf][v * NB + bj] = a[ku][v];
+                if (in_col) sh.recip[buf] = recip;
             }
+            if (in_col) {
 #pragma unroll
-        for (int v = 0; v < BS; ++v)
-            if (j0 + v == k) {
-#pragma unroll
-                for (int u = 0; u < BS; ++u) sh.col[buf][i0 + u] = a[u][v];
+                for (int u = 0; u < BS; ++u) sh.col[buf][u * NB + bi] = a[u][ku];
             }
-        __syncthreads();
-        const double piv = sh.row[buf][k].re;
-        if (!(piv > floor)) return false;  // uniform: every thread reads the same pivot
-        const double p = 1.0 / piv;
-        Cd rj[BS], cp[BS];
+            __syncthreads();
+            const double piv = sh.row[buf][ku * NB + kb].re;
+            const double p = sh.recip[buf];
+            Cd rj[BS], cp[BS];
 #pragma unroll
-        for (int v = 0; v < BS; ++v) rj[v] = sh.row[buf][j0 + v];
+            for (int v = 0; v < BS; ++v) rj[v] = sh.row[buf][v * NB + bj];
 #pragma unroll
-        for (int u = 0; u < BS; ++u) {
-            const Cd ci = sh.col[buf][i0 + u];
-            cp[u] = Cd{ci.re * p, ci.im * p};
-        }
-        // every entry: a_ij - a_ik a_kj / a_kk
-#pragma unroll
-        for (int u = 0; u < BS; ++u)
-#pragma unroll
-            for (int v = 0; v < BS; ++v) {
-                const double gre =
-                    fma(-cp[u].re, rj[v].re, fma(cp[u].im, rj[v].im, a[u][v].re));
-                const double gim =
-                    fma(-cp[u].re, rj[v].im, fma(-cp[u].im, rj[v].re, a[u][v].im));
-                a[u][v] = Cd{gre, gim};
+            for (int u = 0; u < BS; ++u) {
+                const Cd ci = sh.col[buf][u * NB + bi];
+                cp[u] = Cd{ci.re * p, ci.im * p};
             }
-        // then the pivot row (a_kj / a_kk; the pivot 1 / a_kk) and the pivot
-        // column (-a_ik / a_kk) over what the line above wrote there: only
-        // the threads holding row or column k take these branches
+            if (!(piv > floor)) return false;  // uniform: every thread reads the same pivot
+            // every entry: a_ij - a_ik a_kj / a_kk
 #pragma unroll
-        for (int u = 0; u < BS; ++u)
-            if (i0 + u == k) {
+            for (int u = 0; u < BS; ++u)
+#pragma unroll
+                for (int v = 0; v < BS; ++v) {
+                    const double gre =
+                        fma(-cp[u].re, rj[v].re, fma(cp[u].im, rj[v].im, a[u][v].re));
+                    const double gim =
+                        fma(-cp[u].re, rj[v].im, fma(-cp[u].im, rj[v].re, a[u][v].im));
+                    a[u][v] = Cd{gre, gim};
+                }
+            recip = 1.0 / a[(ku + 1) % BS][(ku + 1) % BS].re;
+            // then the pivot row (a_kj / a_kk; the pivot 1 / a_kk) and the pivot
+            // column (-a_ik / a_kk) over what the lines above wrote there
+            if (in_row) {
 #pragma unroll
                 for (int v = 0; v < BS; ++v)
-                    a[u][v] = j0 + v == k ? Cd{p, 0.0} : Cd{rj[v].re * p, rj[v].im * p};
+                    a[ku][v] = in_col && v == ku ? Cd{p, 0.0} : Cd{rj[v].re * p, rj[v].im * p};
             }
-#pragma unroll
-        for (int v = 0; v < BS; ++v)
-            if (j0 + v == k) {
+            if (in_col) {
 #pragma unroll
                 for (int u = 0; u < BS; ++u)
-                    if (i0 + u != k) a[u][v] = Cd{-cp[u].re, -cp[u].im};
+                    if (!(in_row && u == ku)) a[u][ku] = Cd{-cp[u].re, -cp[u].im};
             }
+        }
     }
     return true;
 }
