@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -47,18 +48,23 @@ struct bf_doa {
     double* d_capon = nullptr;
     double* d_bart = nullptr;
     int* d_ok = nullptr;
-    double* d_broadband = nullptr;
+    // One allocation, read with one copy: broadband [2][n], peaks
+    // [2][max_peaks][2], and their counts [2] (int) at the end.
+    double* d_results = nullptr;
     double* d_peaks = nullptr;
     int* d_npeaks = nullptr;
+    double* h_results = nullptr;  // pinned; one reader at a time
+    std::mutex read_mu;
+    size_t results_count() const { return 2 * cfg.n_theta + 4 * cfg.max_peaks + 1; }
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};  // around the 3 kernels
 
     ~bf_doa() {
         for (hipEvent_t e : ev)
             if (e) (void)hipEventDestroy(e);
         for (void* p : {(void*)d_freqs, (void*)d_theta, (void*)d_sin, (void*)d_rs, (void*)d_state,
-                        (void*)d_capon, (void*)d_bart, (void*)d_ok, (void*)d_broadband,
-                        (void*)d_peaks, (void*)d_npeaks})
+                        (void*)d_capon, (void*)d_bart, (void*)d_ok, (void*)d_results})
             if (p) (void)hipFree(p);
+        if (h_results) (void)hipHostFree(h_results);
     }
     void sync() {
         hip_check(hipStreamSynchronize(last_stream), "hipStreamSynchronize");
@@ -119,9 +125,12 @@ bf_status bf_doa_create(const bf_doa_config* c, bf_doa** out) {
         d->d_capon = dmalloc<double>(F * n);
         d->d_bart = dmalloc<double>(F * n);
         d->d_ok = dmalloc<int>(F);
-        d->d_broadband = dmalloc<double>(2 * n);
-        d->d_peaks = dmalloc<double>(2 * c->max_peaks * 2);
-        d->d_npeaks = dmalloc<int>(2);
+        d->d_results = dmalloc<double>(d->results_count());
+        d->d_peaks = d->d_results + 2 * n;
+        d->d_npeaks = reinterpret_cast<int*>(d->d_peaks + 4 * c->max_peaks);
+        hip_check(hipHostMalloc(reinterpret_cast<void**>(&d->h_results),
+                                d->results_count() * sizeof(double), hipHostMallocDefault),
+                  "hipHostMalloc results");
         for (hipEvent_t& e : d->ev) hip_check(hipEventCreate(&e), "hipEventCreate");
         *out = d.release();
     });
@@ -156,7 +165,7 @@ bf_status bf_doa_update(bf_doa* d, void* stream, const uint8_t* x, size_t n_time
                              d->d_ok);
         hip_check(hipEventRecord(d->ev[2], s), "hipEventRecord");
         launch_doa_estimate(s, d->d_capon, d->d_bart, c.n_freq, c.n_theta, d->d_theta,
-                            c.max_peaks, d->d_broadband, d->d_peaks, d->d_npeaks);
+                            c.max_peaks, d->d_results, d->d_peaks, d->d_npeaks);
         hip_check(hipEventRecord(d->ev[3], s), "hipEventRecord");
         d->initialised = true;
         d->last_stream = s;
@@ -182,19 +191,17 @@ bf_status bf_doa_last_timings(bf_doa* d, bf_doa_timings* t) {
 bf_status bf_doa_read_results(bf_doa* d, double* broadband, double* peaks, int* n_peaks) {
     return guarded([&] {
         require_ptr(d, "doa");
+        const size_t n = d->cfg.n_theta, np = 4 * d->cfg.max_peaks;
+        std::lock_guard<std::mutex> lock(d->read_mu);
+        // behind the update on its stream; three copies into pageable memory
+        // cost 25 us each
+        hip_check(hipMemcpyAsync(d->h_results, d->d_results, d->results_count() * sizeof(double),
+                                 hipMemcpyDeviceToHost, d->last_stream),
+                  "hipMemcpyAsync results");
         d->sync();
-        const size_t n = d->cfg.n_theta;
-        if (broadband)
-            hip_check(hipMemcpy(broadband, d->d_broadband, 2 * n * sizeof(double),
-                                hipMemcpyDeviceToHost),
-                      "hipMemcpy broadband");
-        if (peaks)
-            hip_check(hipMemcpy(peaks, d->d_peaks, 4 * d->cfg.max_peaks * sizeof(double),
-                                hipMemcpyDeviceToHost),
-                      "hipMemcpy peaks");
-        if (n_peaks)
-            hip_check(hipMemcpy(n_peaks, d->d_npeaks, 2 * sizeof(int), hipMemcpyDeviceToHost),
-                      "hipMemcpy n_peaks");
+        if (broadband) std::memcpy(broadband, d->h_results, 2 * n * sizeof(double));
+        if (peaks) std::memcpy(peaks, d->h_results + 2 * n, np * sizeof(double));
+        if (n_peaks) std::memcpy(n_peaks, d->h_results + 2 * n + np, 2 * sizeof(int));
     });
 }
 
