@@ -52,7 +52,7 @@ struct OptGridArgs {
 };
 
 // Windows whose operands are prepared together at most.
-inline constexpr int kOptBatch = 4;
+inline constexpr int kOptBatch = 8;
 
 // Scan operands of `n` <= kOptBatch consecutive windows, per channel:
 // operand_bytes each, the trace, and the form (1: R^-1 in FP64; 0: R in

@@ -87,7 +87,7 @@ struct bf_opt_tracker {
     // and factor of the next batch run on the prep stream while this one's
     // windows are searched.
     OptWindows slot[2];
-    int* d_rs = nullptr;  // [kOptBatch][F][M][M][2], of the batch in preparation
+    int* d_rs = nullptr;  // [windows][F][M][M][2], of the batch in preparation
     hipStream_t prep = nullptr;
     // ev_done: the end of the last run on its stream; the next run's stream
     // (which may be another one) waits on it before it writes any state.
@@ -186,13 +186,15 @@ struct bf_opt_tracker {
         // The prep stream starts after the caller's prior work (the input).
         hip_check(hipEventRecord(ev_start, stream), "hipEventRecord");
         hip_check(hipStreamWaitEvent(prep, ev_start, 0), "hipStreamWaitEvent");
-        // Batches of kOptBatch windows, after a first one of a single window,
-        // whose preparation nothing hides.
+        // Batches of 1, 2, 4 and then kOptBatch windows: nothing hides the
+        // preparation of the first, a short search little of the second's, and
+        // every batch costs the events between the streams (against batches of
+        // 1, 4, 4, ...: 48 Bartlett windows 4 % faster, 10 Capon windows equal).
         size_t begin = 0;
         for (size_t batch = 0; begin < W; ++batch) {
             const int k = (int)(batch & 1);
             OptWindows& q = slot[k];
-            q.n = batch == 0 ? 1 : std::min<size_t>(kOptBatch, W - begin);
+            q.n = std::min(std::min<size_t>(kOptBatch, W - begin), (size_t)1 << std::min<size_t>(batch, 16));
             // prep: the batch's operands into slot k, once the search of the
             // batch before the last has released it
             if (batch >= 2)
@@ -305,12 +307,13 @@ void create_tracker(const float* positions, const float* frequencies, const bf_d
     hip_check(hipMemcpy(t->d_freqs, fr.data(), F * sizeof(float), hipMemcpyHostToDevice),
               "hipMemcpy frequencies");
     t->d_state = dmalloc<double>(F * M * M * 2);
+    const size_t batch = std::min<size_t>(kOptBatch, ceil_div(d.n_time, c->integration_spectra));
     for (OptWindows& q : t->slot) {
-        q.operand = dmalloc<char>(kOptBatch * F * opt_operand_bytes(M, t->capon));
-        q.trace = dmalloc<double>(kOptBatch * F);
-        q.mode = dmalloc<int>(kOptBatch * F);
+        q.operand = dmalloc<char>(batch * F * opt_operand_bytes(M, t->capon));
+        q.trace = dmalloc<double>(batch * F);
+        q.mode = dmalloc<int>(batch * F);
     }
-    t->d_rs = dmalloc<int>(kOptBatch * F * M * M * 2);
+    t->d_rs = dmalloc<int>(batch * F * M * M * 2);
     // default priority (a stream of another priority is never created here)
     hip_check(hipStreamCreateWithFlags(&t->prep, hipStreamNonBlocking), "hipStreamCreate");
     for (hipEvent_t* e : {&t->ev_done, &t->ev_start, &t->ev_ready[0], &t->ev_ready[1], &t->ev_used[0],
