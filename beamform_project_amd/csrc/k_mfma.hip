@@ -113,7 +113,10 @@ void launch_mfma_fused(hipStream_t stream, bool split, const uint8_t* x, const f
         if (it != tune_cache().end()) cfg = it->second;
     }
     const MfmaLaunch L{x, w, out, mask, (int)T, (int)F, (int)B, (int)S, split ? 2 : 1};
-    if (!launch_cfg(stream, L, (int)A, cfg)) invalid("MFMA tile shape is not instantiated");
+    if (frame_wave_supported(L, (int)A))
+        launch_frame_wave(stream, L);
+    else if (!launch_cfg(stream, L, (int)A, cfg))
+        invalid("MFMA tile shape is not instantiated");
     hip_check(hipGetLastError(), "mfma_fused_kernel launch");
 }
 
@@ -173,8 +176,12 @@ std::vector<MfmaTuneResult> autotune_mfma_fused(hipStream_t stream, bool split,
             std::lock_guard<std::mutex> lock(g_tune_mu);
             tune_cache()[TuneKey((int)T, (int)F, (int)A, (int)B, (int)S, split)] = best->cfg;
         }
-        // the output ends with the winner's result (every shape computes the same sums)
-        launch_cfg(stream, L, (int)A, best->cfg);
+        // the output ends with what a launch gives (every shape computes the
+        // same sums; the kernel without shapes takes its problems regardless)
+        if (frame_wave_supported(L, (int)A))
+            launch_frame_wave(stream, L);
+        else
+            launch_cfg(stream, L, (int)A, best->cfg);
         hip_check(hipGetLastError(), "mfma_fused_kernel launch");
         hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
     }

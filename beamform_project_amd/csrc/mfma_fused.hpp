@@ -610,6 +610,10 @@ void launch_split_db(hipStream_t stream, const MfmaLaunch& L, const MfmaConfig& 
 
 }  // namespace mfma_detail
 
+// The kernel of k_mfma_wave.hip, where it takes the problem.
+bool frame_wave_supported(const MfmaLaunch& L, int A);
+void launch_frame_wave(hipStream_t stream, const MfmaLaunch& L);
+
 // Launches the kernel with float weights (PARTS = 3) for `A` antennas
 // (k_mfma_exact.hip): `L.tiled` chooses the weight layout.
 void launch_mfma_exact(hipStream_t stream, const MfmaLaunch& L, int A);

@@ -50,7 +50,9 @@ def test_float_weights_vs_fp64(T, A, B, S):
 
 @pytest.mark.parametrize("kernel,tol", [(K.SPLIT_F16, 1e-5), (K.F16, 2e-3)])
 @pytest.mark.parametrize("T,A,B,S", [(1, 64, 9, 64), (64, 32, 40, 64), (65, 128, 12, 64),
-                                     (1285, 64, 100, 320), (961, 256, 45, 320)])
+                                     (1285, 64, 100, 320), (961, 256, 45, 320),
+                                     (17, 256, 1, 64), (195, 256, 48, 64), (195, 256, 49, 64),
+                                     (700, 256, 9, 128)])
 def test_long_windows_vs_fp64(kernel, tol, T, A, B, S):
     x, w = random_case(T, A, B, seed=3 * T + B)
     got = run_gpu(kernel, x, w, api.Dimensions(T, F, A, B), S)
