@@ -443,7 +443,8 @@ def tracker_cpu_baseline(seconds, B, F_):
             O.beam_tracker(x, T, F0, A, 0.0, 0.0, 1e-5, 0.0, S, threads=True)
         return time.perf_counter() - t0
 
-    T, med = median_of_five(run, S, S, seconds)
+    # the trajectory must stay on the sky: T 1e-5 < 1
+    T, med = median_of_five(run, S, S, seconds, hi=90000 // S * S)
     return {"value": round(T * F0 / med, 1), "unit": "beam-samples/s", "cores": threads,
             "kind": "reference" if R is not None else "port",
             "sample": f"beam_tracker_opt_v2 (OpenMP), one beam, T={T} x F={F0}, A={A}, "
