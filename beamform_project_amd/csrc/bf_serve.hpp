@@ -74,7 +74,7 @@ struct ServeLaunch {
     ServeCtrl* ctrl = nullptr;
     ServeWork* work = nullptr;
     const long long* heads = nullptr;  // device view of the pinned head ring
-    int grid = 0;  // persistent workgroups of the item kernel
+    int grid = 0;  // persistent workgroups of the task kernel
     bool split = true;
 };
 
@@ -85,7 +85,7 @@ inline int serve_windows_per_item(int S) {
     return w < 1 ? 1 : w;
 }
 
-// The step: plan kernel + item kernel (capturable; the head comes from the
+// The step: plan kernel + task kernel (capturable; the head comes from the
 // pinned ring, so the captured launch never changes).
 void launch_serve_step(hipStream_t stream, const ServeLaunch& launch);
 

@@ -27,7 +27,7 @@
 //                   level the window's direction.  (A launch of its own for
 //                   the decision costs two more gaps per level; letting the
 //                   last workgroup decide costs each one a fence across the
-//                   XCDs, 105 us instead of 13 for 144 cells.)
+//                   XCDs, 105 us instead of 23 for 144 cells.)
 // Level 0 scans the G x G grid centred on the previous estimate
 // (build_centred_grid, :798-828); each refinement level scans the 3 x 3
 // neighbourhood of the running centre at half the previous pitch
