@@ -206,7 +206,9 @@ void mfma_fused_kernel(
     const bool has_beams = beam0 < B;
 
     bf_half8 bw[PARTS][NT][KS];
-    if (has_beams) load_weights<A, NT, PARTS>(w, tiled, F, B, f, beam0, lane, bw);
+    // only float weights come tiled: a fixed stride lets the loads merge
+    if (has_beams)
+        load_weights<A, NT, PARTS>(w, PARTS == 3 && tiled, F, B, f, beam0, lane, bw);
 
     const int tile_begin = chunk * tiles_per_chunk;
     int tile_end = tile_begin + tiles_per_chunk;
