@@ -45,6 +45,7 @@
 
 #include "bf_doa.hpp"
 #include "gauss_jordan.hpp"
+#include "opt_decide.hpp"
 #include "steering.hpp"
 
 namespace bfhip {
@@ -448,40 +449,20 @@ struct ScanArgs {
     float* dirs;
 };
 
-constexpr int kScanWaves = 8;
-constexpr int kScanThreads = 64 * kScanWaves;
-
 // The decision on the launch before, by the whole workgroup: its powers summed
-// over the channel groups, in FP64 and a fixed order (`ways` threads per cell,
-// their partial sums in LDS), then thread 0's serial part; the new state goes
-// to *out.  P and sums: LDS scratch.
+// over the channel groups (opt_decide.hpp), then thread 0's serial part; the
+// new state goes to *out.  LDS scratch: P[before_cells], sums[kScanThreads].
 __device__ void decide(const ScanArgs& a, float* P, double* sums, OptSearch* out) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int n_cells = a.before_cells;
-    const int padded = (n_cells + 15) & ~15;
+    const int groups = a.before_groups;
     const int level = a.before_level, last_level = a.last_level;
     const OptGridArgs& g = a.g;
-    const int ways = padded < kScanThreads ? kScanThreads / padded : 1;
-    const int per = (a.before_groups + ways - 1) / ways;
-    for (int i = tid; i < padded * ways; i += kScanThreads) {
-        const int cell = i % padded, way = i / padded;
-        const int end = min(a.before_groups, (way + 1) * per);
-        double sum = 0.0;
-#pragma unroll 8
-        for (int q = way * per; q < end; ++q) sum += a.before_part[(size_t)q * padded + cell];
-        if (ways > 1)
-            sums[i] = sum;
-        else
-            P[cell] = (float)sum;
-    }
+    decide_sum(tid, n_cells, groups, a.before_part, P, sums);
     __syncthreads();
-    if (ways > 1) {
-        for (int cell = tid; cell < n_cells; cell += kScanThreads) {
-            double sum = 0.0;
-            for (int way = 0; way < ways; ++way) sum += sums[way * padded + cell];
-            P[cell] = (float)sum;
-        }
+    if (decide_split(n_cells, groups).ways > 1) {
+        decide_fold(tid, n_cells, groups, sums, P);
         __syncthreads();
     }
     if (tid >= 64) return;
