@@ -95,38 +95,72 @@ __device__ __forceinline__ bf_float4 mfma_16x16x32(bf_half8 a, bf_half8 b, bf_fl
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
-// Slice q of the weight component e, as the 16 bits of its operand element.
-// Bfloat16 slices are cut off, not rounded: 8 + 8 + 8 bits hold all 24 of
+// The three bfloat16 slices of the weight component e, as the 16 bits of
+// their operand elements: cut off, not rounded, 8 + 8 + 8 bits hold all 24 of
 // a float.  Infinities and NaN stay whole in slice 0.
-template <int PARTS>
-__device__ __forceinline__ void weight_slices(float e, _Float16 (&out)[PARTS]) {
-    if constexpr (PARTS == 3) {
-        auto top = [](float v) { return __builtin_bit_cast(unsigned, v) & 0xFFFF0000u; };
-        auto bits = [](unsigned u) {
-            return __builtin_bit_cast(_Float16, (unsigned short)(u >> 16));
-        };
-        unsigned h = top(e);
-        float r = e - __builtin_bit_cast(float, h);
-        if (!isfinite(e)) {
-            r = 0.0f;
-            if (isnan(e)) h |= 0x00400000u;  // a NaN of low payload bits only stays a NaN
+__device__ __forceinline__ void weight_slices(float e, _Float16 (&out)[3]) {
+    auto top = [](float v) { return __builtin_bit_cast(unsigned, v) & 0xFFFF0000u; };
+    auto bits = [](unsigned u) { return __builtin_bit_cast(_Float16, (unsigned short)(u >> 16)); };
+    unsigned h = top(e);
+    float r = e - __builtin_bit_cast(float, h);
+    if (!isfinite(e)) {
+        r = 0.0f;
+        if (isnan(e)) h |= 0x00400000u;  // a NaN of low payload bits only stays a NaN
+    }
+    const unsigned m = top(r);
+    out[0] = bits(h);
+    out[1] = bits(m);
+    out[2] = bits(top(r - __builtin_bit_cast(float, m)));
+}
+
+// Loads the B operand (weights) of one wave into registers, from canonical
+// [B][F][A]: fp16 weights, whole vectors of both slices at a time.
+template <int A, int NT, int PARTS>
+__device__ __forceinline__ void load_weights(const float2* __restrict__ w, int F, int B, int f,
+                                             int beam0, int lane, bf_half8 (&bhi)[NT][A / 16],
+                                             bf_half8 (&blo)[NT][A / 16]) {
+    static_assert(PARTS <= 2, "fp16 slices");
+    constexpr int KS = A / 16;
+    const int c = lane & 15;
+    const int g = lane >> 4;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const int b = beam0 + nt * 8 + (c >> 1);
+        const bool comp_im = (c & 1) != 0;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            bf_half8 h, l;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int a = g * (A / 4) + 4 * s + j;
+                float2 v = make_float2(0.0f, 0.0f);
+                if (b < B) v = w[((size_t)b * F + f) * A + a];
+                // column re: (wr, -wi); column im: (wi, wr)
+                const float e0 = comp_im ? v.y : v.x;
+                const float e1 = comp_im ? v.x : -v.y;
+                const _Float16 h0 = (_Float16)e0;
+                const _Float16 h1 = (_Float16)e1;
+                h[2 * j] = h0;
+                h[2 * j + 1] = h1;
+                if (PARTS == 2) {
+                    l[2 * j] = (_Float16)(e0 - (float)h0);
+                    l[2 * j + 1] = (_Float16)(e1 - (float)h1);
+                }
+            }
+            bhi[nt][s] = h;
+            if (PARTS == 2) blo[nt][s] = l;
         }
-        const unsigned m = top(r);
-        out[0] = bits(h);
-        out[1] = bits(m);
-        out[2] = bits(top(r - __builtin_bit_cast(float, m)));
-    } else {
-        out[0] = (_Float16)e;
-        if constexpr (PARTS == 2) out[1] = (_Float16)(e - (float)out[0]);
     }
 }
 
-// Loads the B operand (weights) of one wave into registers: canonical
-// [B][F][A], or tiled [F][B/32][A][32].
-template <int A, int NT, int PARTS>
-__device__ __forceinline__ void load_weights(const float2* __restrict__ w, bool tiled, int F,
-                                             int B, int f, int beam0, int lane,
-                                             bf_half8 (&bw)[PARTS][NT][A / 16]) {
+// The same of float weights, canonical or tiled [F][B/32][A][32], as three
+// bfloat16 slices.
+template <int A, int NT>
+__device__ __forceinline__ void load_float_weights(const float2* __restrict__ w, bool tiled, int F,
+                                                   int B, int f, int beam0, int lane,
+                                                   bf_half8 (&b0)[NT][A / 16],
+                                                   bf_half8 (&b1)[NT][A / 16],
+                                                   bf_half8 (&b2)[NT][A / 16]) {
     constexpr int KS = A / 16;
     const int c = lane & 15;
     const int g = lane >> 4;
@@ -145,15 +179,15 @@ __device__ __forceinline__ void load_weights(const float2* __restrict__ w, bool 
                 const int a = g * (A / 4) + 4 * s + j;
                 float2 v = make_float2(0.0f, 0.0f);
                 if (b < B) v = wb[a * step];
-                // column re: (wr, -wi); column im: (wi, wr)
-                _Float16 e0[PARTS], e1[PARTS];
-                weight_slices<PARTS>(comp_im ? v.y : v.x, e0);
-                weight_slices<PARTS>(comp_im ? v.x : -v.y, e1);
-#pragma unroll
-                for (int q = 0; q < PARTS; ++q) {
-                    bw[q][nt][s][2 * j] = e0[q];
-                    bw[q][nt][s][2 * j + 1] = e1[q];
-                }
+                _Float16 e0[3], e1[3];
+                weight_slices(comp_im ? v.y : v.x, e0);
+                weight_slices(comp_im ? v.x : -v.y, e1);
+                b0[nt][s][2 * j] = e0[0];
+                b0[nt][s][2 * j + 1] = e1[0];
+                b1[nt][s][2 * j] = e0[1];
+                b1[nt][s][2 * j + 1] = e1[1];
+                b2[nt][s][2 * j] = e0[2];
+                b2[nt][s][2 * j + 1] = e1[2];
             }
         }
     }
@@ -161,15 +195,8 @@ __device__ __forceinline__ void load_weights(const float2* __restrict__ w, bool 
 
 // At least two waves per SIMD (at most 256 registers per lane): the
 // unrolled stage otherwise keeps several tiles' accumulators in flight.
-// Eight-wave groups with 64 registers of weights and one LDS stage run two
-// to a CU within 128 registers (1.02 ms against 1.30 ms at A = 64, T = 32768,
-// B = 128, S = 10 where six registers more leave one group).
-constexpr int min_waves(int A, int NT, int WV, int parts, bool db) {
-    return WV == 8 && !db && parts * NT * A / 4 == 64 ? 4 : 2;
-}
 template <int A, int NT, int WV, int PARTS, int MODE, int ST, bool DB, bool MASKED = false>
-__global__ __launch_bounds__(WV * kWaveSize)
-__attribute__((amdgpu_waves_per_eu(min_waves(A, NT, WV, PARTS, DB))))
+__global__ __launch_bounds__(WV * kWaveSize) __attribute__((amdgpu_waves_per_eu(2)))
 void mfma_fused_kernel(
     const uint8_t* __restrict__ x, const float2* __restrict__ w, bool tiled,
     float* __restrict__ out, const uint8_t* __restrict__ mask, int T, int F, int B, int S, int W,
@@ -205,10 +232,16 @@ void mfma_fused_kernel(
     const int beam0 = (blockIdx.y * WV + wave) * NT * 8;
     const bool has_beams = beam0 < B;
 
-    bf_half8 bw[PARTS][NT][KS];
-    // only float weights come tiled: a fixed stride lets the loads merge
-    if (has_beams)
-        load_weights<A, NT, PARTS>(w, PARTS == 3 && tiled, F, B, f, beam0, lane, bw);
+    // the slices, largest first
+    bf_half8 b0[NT][KS];
+    bf_half8 b1[NT][KS];
+    bf_half8 b2[NT][KS];
+    if (has_beams) {
+        if constexpr (PARTS == 3)
+            load_float_weights<A, NT>(w, tiled, F, B, f, beam0, lane, b0, b1, b2);
+        else
+            load_weights<A, NT, PARTS>(w, F, B, f, beam0, lane, b0, b1);
+    }
 
     const int tile_begin = chunk * tiles_per_chunk;
     int tile_end = tile_begin + tiles_per_chunk;
@@ -437,10 +470,18 @@ void mfma_fused_kernel(
                                  : *reinterpret_cast<const bf_half8*>(
                                        cur + tl * TILE_BYTES + (s * kWaveSize + lane) * 16);
 #pragma unroll
-                    for (int q = 0; q < PARTS; ++q)
+                    for (int nt = 0; nt < NT; ++nt)
+                        acc[nt] = mfma_16x16x32<PARTS>(a_s, b0[nt][s], acc[nt]);
+                    if (PARTS >= 2) {
 #pragma unroll
                         for (int nt = 0; nt < NT; ++nt)
-                            acc[nt] = mfma_16x16x32<PARTS>(a_s, bw[q][nt][s], acc[nt]);
+                            acc[nt] = mfma_16x16x32<PARTS>(a_s, b1[nt][s], acc[nt]);
+                    }
+                    if (PARTS == 3) {
+#pragma unroll
+                        for (int nt = 0; nt < NT; ++nt)
+                            acc[nt] = mfma_16x16x32<PARTS>(a_s, b2[nt][s], acc[nt]);
+                    }
                 }
             }
             if (DB) {
