@@ -149,8 +149,9 @@ void launch_fp32_fused(hipStream_t stream, const uint8_t* x, const float* w,
     const bool pays = B >= 4 ? T * B * A >= 65536 : T >= 2048 && (S > 0 || A > 32);
     if (pays && mfma_supported(A, B, S) && T <= (size_t)INT32_MAX / 8 && S <= (size_t)INT32_MAX / 8 &&
         F <= 65535) {
-        const MfmaLaunch L{x, w, out, nullptr, (int)T, (int)F, (int)B, (int)S, 3,
-                           layout == WeightLayout::Tiled};
+        MfmaLaunch L{x, w, out, nullptr, (int)T, (int)F, (int)B, (int)S, 3,
+                     layout == WeightLayout::Tiled};
+        L.one_by_one = S % 64 == 0;  // (against the FMA kernel; not against groups of four)
         launch_mfma_exact(stream, L, (int)A);
         return;
     }

@@ -69,6 +69,14 @@ MfmaConfig default_config(int A, int B, bool split) {
     return c;
 }
 
+MfmaLaunch problem(bool split, const uint8_t* x, const float* w, float* out, const uint8_t* mask,
+                   size_t T, size_t F, size_t A, size_t B, size_t S) {
+    MfmaLaunch L{x, w, out, mask, (int)T, (int)F, (int)B, (int)S, split ? 2 : 1};
+    L.one_by_one = mfma_detail::windows_one_by_one((int)A, L.parts, L.T, L.F, L.B, L.S,
+                                                   default_config((int)A, (int)B, split));
+    return L;
+}
+
 bool launch_cfg(hipStream_t stream, const MfmaLaunch& L, int A, const MfmaConfig& cfg) {
     switch (A) {
     case 32: return launch_mfma_a32(stream, L, cfg);
@@ -112,7 +120,7 @@ void launch_mfma_fused(hipStream_t stream, bool split, const uint8_t* x, const f
         auto it = tune_cache().find(TuneKey((int)T, (int)F, (int)A, (int)B, (int)S, split));
         if (it != tune_cache().end()) cfg = it->second;
     }
-    const MfmaLaunch L{x, w, out, mask, (int)T, (int)F, (int)B, (int)S, split ? 2 : 1};
+    const MfmaLaunch L = problem(split, x, w, out, mask, T, F, A, B, S);
     if (frame_wave_supported(L, (int)A))
         launch_frame_wave(stream, L);
     else if (!launch_cfg(stream, L, (int)A, cfg))
@@ -126,7 +134,7 @@ std::vector<MfmaTuneResult> autotune_mfma_fused(hipStream_t stream, bool split,
                                                 size_t S, int repeats) {
     check_problem(T, F, A, B, S);
     if (repeats < 1) invalid("repeats must be positive");
-    const MfmaLaunch L{x, w, out, nullptr, (int)T, (int)F, (int)B, (int)S, split ? 2 : 1};
+    const MfmaLaunch L = problem(split, x, w, out, nullptr, T, F, A, B, S);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     hip_check(hipEventCreate(&e0), "hipEventCreate");
     hip_check(hipEventCreate(&e1), "hipEventCreate");

@@ -36,15 +36,15 @@
 //   MODE 0 (no integration): tile i, row 4G+r -> t = 16i + 4G + r
 //   MODE 1 (S == 10): super-tile of 5 tiles, G covers 20 spectra (2 windows)
 //   MODE 2 (S % 4 == 0): super-tile of S/4 tiles, G covers one window
-//   MODE 3 (S % 64 == 0): tiles as in MODE 0; the row groups share every
-//     window and are folded by two shuffles where it closes.  Windows are
-//     this long that a stage of 4 tiles lies inside one, and the work is
-//     whole windows, not groups of four (A = 256, T = 4100, B = 45, S = 320, 13
-//     windows: 437 -> 383 us)
+//   MODE 3 (S % 64 == 0, few windows): tiles as in MODE 0; the row groups
+//     share every window and are folded by two shuffles where it closes.
+//     Windows are this long that a stage of 4 tiles lies inside one, and the
+//     work is whole windows, not groups of four
 // Re and im of a beam sit in adjacent lanes; a quad-permute DPP adds the
 // two squared sums.
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 
 #include "bf_kernels.hpp"
@@ -60,6 +60,10 @@ struct MfmaLaunch {
     int T = 0, F = 0, B = 0, S = 0;
     int parts = 2;       // weight slices: 1 fp16, 2 fp16 hi + lo, 3 bfloat16 (the float itself)
     bool tiled = false;  // weights [F][B/32][A][32] instead of [B][F][A]
+    // windows of a multiple of 64 spectra one after another, not four side by
+    // side: these sum in another order, so this follows from the problem alone
+    // (windows_one_by_one), never from a tile shape or a mask
+    bool one_by_one = false;
 };
 
 // Launch the kernel of `cfg` for one antenna count; false when `cfg` is
@@ -556,11 +560,30 @@ void mfma_fused_kernel(
 
 struct Plan {
     int mode, st, tiles_total, tiles_per_chunk, n_items, per_xcd, beam_blocks, W;
+    double cost;  // modelled time, in tiles
 };
 
-inline Plan make_plan(int T, int F, int B, int S, const MfmaConfig& cfg) {
+// Whether windows of a multiple of 20 spectra (and not of 16) stage five tiles
+// at a time instead of one: fewer barriers per tile, five times the LDS.  Up
+// to 64 antennas that is free (split, S = 20, T = 4100, B = 33: A = 32 69 -> 38
+// us, A = 64 73 -> 61 us).  Above it leaves two workgroups to a CU, which
+// costs nothing where no more were launched (A = 128, T = 512, B = 9, S = 20, 336
+// workgroups: 32 -> 27 us; S = 40, 672 of them: 35 -> 41 us).  Beyond those it
+// pays at 128 for two N-tiles of split weights (T = 4100, B = 33, S = 100: 180
+// -> 141 us; but B = 2 87 -> 112 us, F16 98 -> 106 us) and at 256 in long
+// calls (T = 4100, S = 100, B = 33: 510 -> 448 us; T = 1024, B = 20: 71 -> 80 us), for
+// single weights with one block of beams (T = 4100, S = 20: B = 9 0.88 of the
+// time, B = 33 1.05).  Float weights were measured with five tiles only.
+inline bool five_tile_stages(int A, int parts, int nt, int T, int B, long workgroups) {
+    if (A <= 64 || parts == 3 || workgroups <= 512) return true;
+    if (A == 128) return parts == 2 && nt >= 2;
+    return T >= 4096 && (parts == 2 || B <= 32);
+}
+
+inline Plan make_plan(int A, int parts, int T, int F, int B, int S, bool one_by_one,
+                      const MfmaConfig& cfg) {
     Plan p{};
-    p.mode = S == 0 ? 0 : (S == 10 ? 1 : (S % 64 == 0 ? 3 : 2));
+    p.mode = S == 0 ? 0 : (S == 10 ? 1 : (one_by_one ? 3 : 2));
     int tiles_per_super = 1;
     if (p.mode == 0) {
         p.st = 4;
@@ -575,7 +598,7 @@ inline Plan make_plan(int T, int F, int B, int S, const MfmaConfig& cfg) {
         p.W = (int)ceil_div((size_t)T, (size_t)S);
     } else {
         tiles_per_super = S / 4;
-        p.st = tiles_per_super % 4 == 0 ? 4 : (tiles_per_super % 5 == 0 ? 5 : 1);
+        p.st = tiles_per_super % 4 == 0 ? 4 : 1;
         p.W = (int)ceil_div((size_t)T, (size_t)S);
     }
     const int rows_super = 16 * tiles_per_super;
@@ -596,22 +619,58 @@ inline Plan make_plan(int T, int F, int B, int S, const MfmaConfig& cfg) {
         const long chunks = (long)ceil_div((size_t)p.tiles_total, (size_t)c);
         const long rounds =
             (long)ceil_div((size_t)(chunks * F * p.beam_blocks), (size_t)resident);
-        const long cost = rounds * (c + startup_tiles);
+        // A chunk of whole windows may reach past the last tile.  Counted in
+        // full it gives way to more and shorter ones, which measured faster
+        // but for 256 antennas, whose weights weigh more (F16, T = 1024, B =
+        // 128, S = 320: 171 us in two chunks, 142 in one).
+        const long tiles = A == 256 ? std::min(c, p.tiles_total) : c;
+        const long cost = rounds * (tiles + startup_tiles);
         if (best_cost < 0 || cost < best_cost) {
             best_cost = cost;
             per_chunk = c;
+            // the end of a window that runs alone costs about 0.8 tiles
+            p.cost = (double)cost + (p.mode == 3 ? rounds * tiles * 0.8 * 16 / S : 0.0);
         }
     }
     p.tiles_per_chunk = per_chunk;
     const int n_chunks = (int)ceil_div((size_t)p.tiles_total, (size_t)per_chunk);
     p.n_items = n_chunks * F;
     p.per_xcd = (int)ceil_div((size_t)p.n_items, kXcds);
+    if (p.mode == 2 && p.st == 1 && tiles_per_super % 5 == 0 &&
+        five_tile_stages(A, parts, cfg.nt, T, B, (long)p.n_items * p.beam_blocks))
+        p.st = 5;
     return p;
+}
+
+// Whether windows of a multiple of 64 spectra run one after another (MODE 3)
+// instead of four side by side (MODE 2), for the problem's untuned shape
+// `cfg`.  Side by side pads the time axis to whole groups of four windows; one
+// by one costs the folds and stores at the end of every window, 1.5 tiles (24
+// spectra) a window at most.  So one by one where the padding is the larger
+// part: A = 64, split, B = 64, S = 320, T = 512 (2.5 times its length padded) 29
+// -> 16 us, T = 4100 (1.25) 123 -> 102 us; but S = 64, T = 16384 (no padding) 251
+// -> 271 us, and A = 32, B = 2 there 82 -> 108 us.  For 64 and 128 antennas also
+// where shorter chunks fill the chip (A = 64, T = 1024, B = 9, S = 64, 336
+// workgroups against 1008: 24 -> 17 us) or the two are modelled alike (A =
+// 128, T = 8192, B = 9, S = 128: 265 -> 212 us; within 5 %, the least that keeps
+// these); the other counts gain nothing there (A = 32, T = 8192, B = 9, S = 64: 1.16).
+inline bool windows_one_by_one(int A, int parts, int T, int F, int B, int S,
+                               const MfmaConfig& cfg) {
+    if (S == 0 || S % 64 != 0) return false;
+    const long group = 4L * S;
+    const long padding = (T + group - 1) / group * group - T;
+    if (padding * S > 24L * T) return true;
+    if (A != 64 && A != 128) return false;
+    const Plan side = make_plan(A, parts, T, F, B, S, false, cfg);
+    const Plan one = make_plan(A, parts, T, F, B, S, true, cfg);
+    if ((long)side.n_items * side.beam_blocks < cfg.resident && one.n_items > side.n_items)
+        return true;
+    return one.cost < 1.05 * side.cost;
 }
 
 template <int A, int NT, int WV, int PARTS, bool DB, bool MASKED = false>
 void launch_shape(hipStream_t stream, const MfmaLaunch& L, const MfmaConfig& cfg) {
-    const Plan p = make_plan(L.T, L.F, L.B, L.S, cfg);
+    const Plan p = make_plan(A, PARTS, L.T, L.F, L.B, L.S, L.one_by_one, cfg);
     const dim3 grid((unsigned)(p.per_xcd * kXcds), (unsigned)p.beam_blocks);
     const dim3 block(WV * kWaveSize);
     const float2* w2 = reinterpret_cast<const float2*>(L.w);

@@ -52,9 +52,26 @@ def test_float_weights_vs_fp64(T, A, B, S):
 @pytest.mark.parametrize("T,A,B,S", [(1, 64, 9, 64), (64, 32, 40, 64), (65, 128, 12, 64),
                                      (1285, 64, 100, 320), (961, 256, 45, 320),
                                      (17, 256, 1, 64), (195, 256, 48, 64), (195, 256, 49, 64),
-                                     (700, 256, 9, 128)])
+                                     (700, 256, 9, 128),
+                                     # four windows side by side where that pads little, one
+                                     # by one where it pads much, on both sides of the line
+                                     (256, 64, 20, 64), (197, 32, 9, 64), (180, 32, 9, 64),
+                                     (1010, 128, 17, 64), (468, 64, 120, 128),
+                                     (430, 64, 120, 128), (515, 256, 50, 64)])
 def test_long_windows_vs_fp64(kernel, tol, T, A, B, S):
     x, w = random_case(T, A, B, seed=3 * T + B)
+    got = run_gpu(kernel, x, w, api.Dimensions(T, F, A, B), S)
+    ref = fp64_reference(x, w, T, A, B, S)
+    assert rel_err_floored(got, ref, incoherent_floor(x, A, S)) <= tol
+
+
+@pytest.mark.parametrize("kernel,tol", [(K.SPLIT_F16, 1e-5), (K.F16, 2e-3)])
+@pytest.mark.parametrize("T,A,B,S", [(163, 128, 32, 20), (163, 128, 33, 20), (410, 64, 12, 100),
+                                     (301, 256, 9, 20), (4095, 256, 2, 20), (4097, 256, 2, 20),
+                                     (4097, 256, 33, 100)])
+def test_stage_lengths_vs_fp64(kernel, tol, T, A, B, S):
+    """Windows of a multiple of 20 on both sides of the rule for their stages."""
+    x, w = random_case(T, A, B, seed=5 * T + B)
     got = run_gpu(kernel, x, w, api.Dimensions(T, F, A, B), S)
     ref = fp64_reference(x, w, T, A, B, S)
     assert rel_err_floored(got, ref, incoherent_floor(x, A, S)) <= tol
