@@ -51,12 +51,25 @@ __device__ __forceinline__ void load_block_weights(const float2* __restrict__ w,
     }
 }
 
+// One tile in flight.  With a loss mask the row's byte travels beside its
+// voltages and clears them where they are used, so that neither load waits for
+// the other.
+template <bool MASKED>
+struct Tile {
+    TileBytes<kA> bytes;
+};
+template <>
+struct Tile<true> {
+    TileBytes<kA> bytes;
+    uint8_t valid;
+};
+
 // Windows [w_begin, w_end) of one channel for 8 beams per wave.
-template <int PARTS>
+template <int PARTS, bool MASKED>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void frame_wave_kernel(const uint8_t* __restrict__ x, const float2* __restrict__ w,
-                       float* __restrict__ out, int T, int F, int B, int S, int W, int run,
-                       int blocks, long n_tasks, int per_xcd) {
+                       float* __restrict__ out, const uint8_t* __restrict__ mask, int T, int F,
+                       int B, int S, int W, int run, int blocks, long n_tasks, int per_xcd) {
     const long group = (long)(blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
     const long task = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWaveSize)) +
                       group * kWaves;
@@ -80,21 +93,28 @@ void frame_wave_kernel(const uint8_t* __restrict__ x, const float2* __restrict__
     const int tile_last = min(w_end * (S >> 4), (T + 15) >> 4);  // exclusive
     const int per_window = S >> 4;
     // Tile i: rows 16 i .. 16 i + 15; rows at or after T read as zero.
-    auto load_tile = [&](int i) -> TileBytes<kA> {
+    auto load_tile = [&](int i) -> Tile<MASKED> {
         const uint8_t* const p = x_f + (size_t)i * 16 * row_stride;
-        if (16 * (i + 1) <= T) return load_bytes<kA>(p + lane_off);
-        TileBytes<kA> r;
+        const int t = 16 * i + col;
+        Tile<MASKED> r;
+        if constexpr (MASKED) r.valid = t < T ? mask[(size_t)t * F + f] : 0;
+        if (16 * (i + 1) <= T) {
+            r.bytes = load_bytes<kA>(p + lane_off);
+            return r;
+        }
 #pragma unroll
-        for (int s = 0; s < kSteps; ++s) r.w[s] = 0u;
-        if (16 * i + col < T) r = load_bytes<kA>(p + lane_off);
+        for (int s = 0; s < kSteps; ++s) r.bytes.w[s] = 0u;
+        if (t < T) r.bytes = load_bytes<kA>(p + lane_off);
         return r;
     };
     float win = 0.0f;
-    auto use_tile = [&](const TileBytes<kA>& t) {
+    auto use_tile = [&](const Tile<MASKED>& t) {
+        unsigned keep = ~0u;
+        if constexpr (MASKED) keep = t.valid != 0 ? ~0u : 0u;
         bf_float4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
 #pragma unroll
         for (int s = 0; s < kSteps; ++s) {
-            const bf_uint4v av = int4_slots<PARTS>(t.w[s]);
+            const bf_uint4v av = int4_slots<PARTS>(t.bytes.w[s] & keep);
             // large and small slices in sums of their own: two chains
 #pragma unroll
             for (int q = 0; q < PARTS; ++q) acc[q] = mfma<PARTS>(av, bw[q][s], acc[q]);
@@ -118,7 +138,7 @@ void frame_wave_kernel(const uint8_t* __restrict__ x, const float2* __restrict__
     };
     // two tiles in flight; a window is a multiple of four tiles, so only the
     // run's end can be odd
-    TileBytes<kA> buf[2];
+    Tile<MASKED> buf[2];
     buf[0] = load_tile(tile_begin);
     if (tile_begin + 1 < tile_last) buf[1] = load_tile(tile_begin + 1);
 #pragma unroll 1
@@ -145,19 +165,27 @@ void launch_parts(hipStream_t stream, const MfmaLaunch& L) {
     const size_t per_xcd = ceil_div(ceil_div(n_tasks, kWaves), kXcds);
     if (per_xcd * kXcds > (size_t)INT32_MAX)
         fail(BF_ERR_OVERFLOW, "MFMA beamformer grid exceeds the supported size");
-    hipLaunchKernelGGL((frame_wave_kernel<PARTS>), dim3((unsigned)(per_xcd * kXcds)),
-                       dim3(kThreads), 0, stream, L.x, reinterpret_cast<const float2*>(L.w), L.out,
-                       L.T, L.F, L.B, L.S, W, (int)run, (int)blocks, (long)n_tasks, (int)per_xcd);
+#define BF_LAUNCH(MASKED_)                                                                     \
+    hipLaunchKernelGGL((frame_wave_kernel<PARTS, MASKED_>), dim3((unsigned)(per_xcd * kXcds)), \
+                       dim3(kThreads), 0, stream, L.x, reinterpret_cast<const float2*>(L.w),   \
+                       L.out, L.mask, L.T, L.F, L.B, L.S, W, (int)run, (int)blocks,            \
+                       (long)n_tasks, (int)per_xcd)
+    if (L.mask != nullptr)
+        BF_LAUNCH(true);
+    else
+        BF_LAUNCH(false);
+#undef BF_LAUNCH
 }
 
 }  // namespace
 
 // Up to six blocks: with more, a channel's blocks no longer run together, the
 // rows are read again from HBM, and sharing them through LDS pays (T = 4096, S =
-// 320: B = 48 438 us staged, 362 here; B = 64 452, 442; B = 96 577, 687).
+// 320: B = 48 438 us staged, 362 here; B = 64 452, 442; B = 96 577, 687).  A mask
+// changes nothing in that, so that a masked frame sums as the plain one does
+// (T = 4100, B = 45, S = 320, masked: 766 us staged, 406 here).
 bool frame_wave_supported(const MfmaLaunch& L, int A) {
-    return A == kA && L.S > 0 && L.S % 64 == 0 && L.B <= 48 && L.parts <= 2 &&
-           L.mask == nullptr && !L.tiled;
+    return A == kA && L.S > 0 && L.S % 64 == 0 && L.B <= 48 && L.parts <= 2 && !L.tiled;
 }
 
 void launch_frame_wave(hipStream_t stream, const MfmaLaunch& L) {

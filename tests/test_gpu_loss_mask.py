@@ -42,6 +42,9 @@ def run(kernel, x, w, dims, S, mask=None):
     # windows side by side and one by one; stages of five tiles and of one
     (64, 20, 64, 256, K.SPLIT_F16), (64, 20, 64, 180, K.SPLIT_F16),
     (128, 40, 20, 250, K.SPLIT_F16), (128, 9, 100, 250, K.F16), (256, 60, 128, 300, K.SPLIT_F16),
+    # one wave per block of 8 beams
+    (256, 9, 64, 195, K.SPLIT_F16), (256, 9, 64, 195, K.F16),
+    (256, 45, 320, 700, K.SPLIT_F16), (256, 48, 128, 128, K.F16),
 ])
 def test_masked_equals_zeroed_payload(A, B, S, T, kernel):
     rng = np.random.default_rng(A * 1000 + B)
