@@ -77,7 +77,26 @@ MfmaLaunch problem(bool split, const uint8_t* x, const float* w, float* out, con
     return L;
 }
 
+// The one-wave kernel sums in an order of its own, so the problems it takes
+// run on no other: its one shape, 8 beams on each of 4 waves without LDS
+// stages, and the chunk sizes.
+MfmaConfig default_config(const MfmaLaunch& L, int A) {
+    MfmaConfig c = default_config(A, L.B, L.parts == 2);
+    if (frame_wave_supported(L, A)) {
+        c.nt = 1;
+        c.waves = 4;
+        c.db = 0;
+        c.resident = 512;
+    }
+    return c;
+}
+
 bool launch_cfg(hipStream_t stream, const MfmaLaunch& L, int A, const MfmaConfig& cfg) {
+    if (frame_wave_supported(L, A)) {
+        if (cfg.nt != 1 || cfg.waves != 4 || cfg.db != 0) return false;
+        launch_frame_wave(stream, L, cfg.resident);
+        return true;
+    }
     switch (A) {
     case 32: return launch_mfma_a32(stream, L, cfg);
     case 64: return launch_mfma_a64(stream, L, cfg);
@@ -114,16 +133,14 @@ void launch_mfma_fused(hipStream_t stream, bool split, const uint8_t* x, const f
                        float* out, size_t T, size_t F, size_t A, size_t B, size_t S,
                        const uint8_t* mask) {
     check_problem(T, F, A, B, S);
-    MfmaConfig cfg = default_config((int)A, (int)B, split);
+    const MfmaLaunch L = problem(split, x, w, out, mask, T, F, A, B, S);
+    MfmaConfig cfg = default_config(L, (int)A);
     {
         std::lock_guard<std::mutex> lock(g_tune_mu);
         auto it = tune_cache().find(TuneKey((int)T, (int)F, (int)A, (int)B, (int)S, split));
         if (it != tune_cache().end()) cfg = it->second;
     }
-    const MfmaLaunch L = problem(split, x, w, out, mask, T, F, A, B, S);
-    if (frame_wave_supported(L, (int)A))
-        launch_frame_wave(stream, L);
-    else if (!launch_cfg(stream, L, (int)A, cfg))
+    if (!launch_cfg(stream, L, (int)A, cfg))
         invalid("MFMA tile shape is not instantiated");
     hip_check(hipGetLastError(), "mfma_fused_kernel launch");
 }
@@ -141,7 +158,7 @@ std::vector<MfmaTuneResult> autotune_mfma_fused(hipStream_t stream, bool split,
     std::vector<MfmaTuneResult> results;
     try {
         // Bring the clocks up before the first candidate is timed.
-        const MfmaConfig warm = default_config((int)A, (int)B, split);
+        const MfmaConfig warm = default_config(L, (int)A);
         for (int r = 0; r < 3; ++r) launch_cfg(stream, L, (int)A, warm);
         hip_check(hipGetLastError(), "mfma_fused_kernel launch");
         for (const auto& sh : shapes_for((int)A)) {
@@ -184,12 +201,8 @@ std::vector<MfmaTuneResult> autotune_mfma_fused(hipStream_t stream, bool split,
             std::lock_guard<std::mutex> lock(g_tune_mu);
             tune_cache()[TuneKey((int)T, (int)F, (int)A, (int)B, (int)S, split)] = best->cfg;
         }
-        // the output ends with what a launch gives (every shape computes the
-        // same sums; the kernel without shapes takes its problems regardless)
-        if (frame_wave_supported(L, (int)A))
-            launch_frame_wave(stream, L);
-        else
-            launch_cfg(stream, L, (int)A, best->cfg);
+        // the output ends with the winner's result (every shape computes the same sums)
+        launch_cfg(stream, L, (int)A, best->cfg);
         hip_check(hipGetLastError(), "mfma_fused_kernel launch");
         hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
     }

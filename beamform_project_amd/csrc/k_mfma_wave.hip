@@ -154,13 +154,14 @@ void frame_wave_kernel(const uint8_t* __restrict__ x, const float2* __restrict__
 }
 
 template <int PARTS>
-void launch_parts(hipStream_t stream, const MfmaLaunch& L) {
+void launch_parts(hipStream_t stream, const MfmaLaunch& L, int resident) {
     const int W = (int)ceil_div((size_t)L.T, (size_t)L.S);
     const size_t blocks = ceil_div((size_t)L.B, 8);
     // windows per task: the weights of one (16 KB) are worth reading once for
     // several, as long as three rounds of the resident waves remain
     const size_t all = (size_t)W * L.F * blocks;
-    const size_t run = std::max<size_t>(1, std::min<size_t>(16, all / 6144));
+    const size_t run =
+        std::max<size_t>(1, std::min<size_t>(16, all / (3 * kWaves * (size_t)resident)));
     const size_t n_tasks = ceil_div((size_t)W, run) * L.F * blocks;
     const size_t per_xcd = ceil_div(ceil_div(n_tasks, kWaves), kXcds);
     if (per_xcd * kXcds > (size_t)INT32_MAX)
@@ -188,11 +189,11 @@ bool frame_wave_supported(const MfmaLaunch& L, int A) {
     return A == kA && L.S > 0 && L.S % 64 == 0 && L.B <= 48 && L.parts <= 2 && !L.tiled;
 }
 
-void launch_frame_wave(hipStream_t stream, const MfmaLaunch& L) {
+void launch_frame_wave(hipStream_t stream, const MfmaLaunch& L, int resident) {
     if (L.parts == 2)
-        launch_parts<2>(stream, L);
+        launch_parts<2>(stream, L, resident);
     else
-        launch_parts<1>(stream, L);
+        launch_parts<1>(stream, L, resident);
 }
 
 }  // namespace bfhip

@@ -712,9 +712,10 @@ void launch_split_db(hipStream_t stream, const MfmaLaunch& L, const MfmaConfig& 
 
 }  // namespace mfma_detail
 
-// The kernel of k_mfma_wave.hip, where it takes the problem.
+// The kernel of k_mfma_wave.hip, where it takes the problem.  `resident`: the
+// workgroups assumed to run at once, which sizes a task's run of windows.
 bool frame_wave_supported(const MfmaLaunch& L, int A);
-void launch_frame_wave(hipStream_t stream, const MfmaLaunch& L);
+void launch_frame_wave(hipStream_t stream, const MfmaLaunch& L, int resident);
 
 // Launches the kernel with float weights (PARTS = 3) for `A` antennas
 // (k_mfma_exact.hip): `L.tiled` chooses the weight layout.

@@ -168,7 +168,9 @@ bf_status bf_resolve_kernel(int kernel, const bf_dims* dims, size_t integration_
  * fastest the shape of every later launch of the same problem (T, F, A, B,
  * S, kernel) in this process.  Synchronous; allocates nothing on the
  * device; leaves a valid result in `output` (every shape computes the same
- * sums).  entries may be NULL; n_entries receives the candidate count. */
+ * sums).  256 antennas with windows of a multiple of 64 spectra and at most
+ * 48 beams run on a kernel without LDS stages: its candidates are the chunk
+ * sizes alone.  entries may be NULL; n_entries receives the candidate count. */
 typedef struct bf_tune_entry {
     int beams_per_wave;
     int waves_per_workgroup;

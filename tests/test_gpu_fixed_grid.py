@@ -399,3 +399,24 @@ def test_autotuned_shapes_compute_identical_sums(T, A, B, S, kernel):
     api.autotune_clear()
     with pytest.raises(_capi.InvalidArgument, match="autotuner"):
         api.autotune_packed_beamformer(K.FP32, None, dx, dw, out, dims, S)
+
+
+@pytest.mark.parametrize("T,B,S,kernel", [(700, 9, 64, K.SPLIT_F16), (650, 45, 320, K.F16)])
+def test_autotuner_times_the_kernel_that_runs(T, B, S, kernel):
+    """256 antennas, long windows and up to 48 beams run on a kernel without LDS
+    stages: the autotuner times that one alone, in its three chunk sizes, and
+    every choice sums as the default does."""
+    A = 256
+    x, w = random_case(T, A, B, seed=T + B)
+    dims = api.Dimensions(T, F, A, B)
+    api.autotune_clear()
+    default = run_gpu(kernel, x, w, dims, S)
+    dx, dw = api.DeviceArray.from_numpy(x), api.DeviceArray.from_numpy(w)
+    out = api.DeviceArray.empty((api.integrated_time_count(T, S), F, B), np.float32)
+    table = api.autotune_packed_beamformer(kernel, None, dx, dw, out, dims, S, repeats=2)
+    shapes = [(r["beams_per_wave"], r["waves_per_workgroup"], r["double_buffered"],
+               r["resident_workgroups"]) for r in table]
+    assert shapes == [(8, 4, 0, 256), (8, 4, 0, 512), (8, 4, 0, 1024)]
+    assert np.array_equal(out.to_numpy(), default)
+    assert np.array_equal(run_gpu(kernel, x, w, dims, S), default)
+    api.autotune_clear()
