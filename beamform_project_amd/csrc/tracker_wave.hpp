@@ -363,9 +363,10 @@ __device__ __forceinline__ TileBytes<A> load_bytes(const uint8_t* p) {
 template <int A>
 constexpr int kDepth = A <= 64 ? 4 : (A == 128 ? 2 : 1);
 // Whether the conversion of a tile runs beside the MFMAs of the one before
-// (two converted operands in registers).
-template <int A>
-constexpr bool kPipelined = A <= 128;
+// (two converted operands in registers).  Masked short windows, which never
+// have a whole group of tiles, leave the code out: with it they ran 11 % slower.
+template <int A, bool ANCHORED, bool MASKED>
+constexpr bool kPipelined = A <= 128 && !(MASKED && ANCHORED);
 
 // Windows [w_begin, w_end) of one channel for the beams beam0 ..
 // beam0 + NT*8 - 1, by one wave (every argument wave-uniform).  The loads of
@@ -459,7 +460,7 @@ __device__ __forceinline__ void wave_windows(const RowSource& rs, const Channel<
         // between the MFMAs of the tile before, where it costs no time.
         int n_fast = 0;
         const long row0 = t_win & rs.ring_mask;
-        if (!MASKED && kPipelined<A>) {
+        if (kPipelined<A, ANCHORED, MASKED>) {
             long full = S >> 4;
             const long room = (rs.t_limit - t_win) >> 4;
             full = full < room ? full : room;
@@ -471,10 +472,28 @@ __device__ __forceinline__ void wave_windows(const RowSource& rs, const Channel<
         }
         const uint8_t* x_next = rs.x_f + (size_t)row0 * rs.row_stride;
         const size_t tile_stride = (size_t)16 * rs.row_stride;
+        // With a loss mask a row's byte travels beside its voltages and clears
+        // them where they are converted: neither load waits for the other.
+        const uint8_t* valid_next =
+            MASKED ? rs.valid_f + (size_t)(row0 + col) * rs.mask_stride : nullptr;
         TileBytes<A> buf[D];
+        uint8_t valid[D];
+        auto load_next = [&](int u) {
+            if (MASKED) valid[u] = valid_next[(size_t)(16 * u) * rs.mask_stride];
+            buf[u] = load_bytes<A>(x_next + u * tile_stride + lane_off);
+        };
+        auto convert_next = [&](int u, bf_uint4v (&av)[KS]) {
+            TileBytes<A> x = buf[u];
+            if (MASKED) {
+                const unsigned keep = valid[u] != 0 ? ~0u : 0u;
+#pragma unroll
+                for (int s = 0; s < KS; ++s) x.w[s] &= keep;
+            }
+            convert(x, av);
+        };
         if (n_fast > 0) {
 #pragma unroll
-            for (int u = 0; u < D; ++u) buf[u] = load_bytes<A>(x_next + u * tile_stride + lane_off);
+            for (int u = 0; u < D; ++u) load_next(u);
         } else {
 #pragma unroll
             for (int u = 0; u < D; ++u)
@@ -486,12 +505,13 @@ __device__ __forceinline__ void wave_windows(const RowSource& rs, const Channel<
             auto group = [&](auto more, int j0) {
                 constexpr bool MORE = decltype(more)::value;
                 x_next += D * tile_stride;
+                if (MASKED) valid_next += (size_t)(16 * D) * rs.mask_stride;
 #pragma unroll
                 for (int u = 0; u < D; ++u) {
                     bf_float4 acc[NT];
                     contract(av[u & 1], acc);
-                    if (MORE) buf[u] = load_bytes<A>(x_next + u * tile_stride + lane_off);
-                    if (MORE || u + 1 < D) convert(buf[(u + 1) % D], av[(u + 1) & 1]);
+                    if (MORE) load_next(u);
+                    if (MORE || u + 1 < D) convert_next((u + 1) % D, av[(u + 1) & 1]);
                     epilogue(j0 + u, acc);
                     if (INTEGRATE) {
 #pragma unroll
@@ -502,7 +522,7 @@ __device__ __forceinline__ void wave_windows(const RowSource& rs, const Channel<
                     }
                 }
             };
-            convert(buf[0], av[0]);
+            convert_next(0, av[0]);
             int j0 = 0;
 #pragma unroll 1
             for (; j0 + D < n_fast; j0 += D) group(std::true_type{}, j0);

@@ -386,6 +386,21 @@ def test_masked_stream_equals_zeroed_payload(stream, mixed):
         assert np.array_equal(ones[i][1], mixed[0][i][1]), f"request {i}"
 
 
+@pytest.mark.parametrize("n_ant,kernel", [(64, K.SPLIT_F16), (32, K.SPLIT_F16), (64, K.F16)])
+def test_masked_window_lengths(stream, n_ant, kernel):
+    """Windows around the length where masked ones take a body of their own (64)
+    and around its groups of four tiles, across the ring's end."""
+    x = np.ascontiguousarray(stream[..., :n_ant])
+    kw = dict(n_ant=n_ant, positions=O.regular_array(n_ant // 8, 8, 0.3), kernel=kernel)
+    requests = [(9, 63, 2300, 0, 0, 20), (9, 64, 2300, 0, 0, 21), (17, 79, 2300, 3, 0, 22),
+                (3, 130, 2200, 41, 0, 23), (20, 255, 2301, 0, 0, 24)]
+    mask = loss_mask(x.shape[0], 5)
+    got, _ = run(requests, x, mask=mask, **kw)
+    want, _ = run(requests, x * mask[:, :, None], **kw)
+    for i in want:
+        assert np.array_equal(got[i][1], want[i][1]), f"request {i}"
+
+
 def test_zero_copy_producer_equals_ingest(stream, mixed):
     # chunks of 100 on a ring of 1024: spans wrap at 1000..1100 and 2000..2100
     got, _ = run(MIX, stream, zero_copy=True)
