@@ -8,9 +8,12 @@
 // 32-bit integer, right to 2^-31 of a turn, after three FP64 FMAs.  Integer
 // operations then split off the quadrant, and the rest, |x| <= pi/4 carried
 // as a float and its remainder, goes through polynomials for sin and cos (to
-// x^7 and x^8: least-maximum fits, off by 1.8e-9 and 5e-11).  The result
-// differs from (float)cos(phi), (float)sin(phi) by about one float ulp, in
-// some 36 instructions where a reduced FP64 phase and sincosf took about 90.
+// x^7 and x^8: least-maximum fits, off by 2.2e-9 and 1.7e-9).  Over random
+// geometries the result is off by at most 8.2e-8 and 1.84e-8 rms, in some 36
+// instructions; a reduced FP64 phase and sincosf took about 90 and were off by
+// 1.00e-7 and 2.14e-8.  Where the caller asks for float weights (the tracker's
+// FP32 selector with several beams or integration) the phase stays in FP64 and
+// the weight is rounded once, off by 2^-25 (cos_sin_turns64).
 #pragma once
 
 #include "bf_tracker.hpp"
@@ -211,6 +214,13 @@ __device__ __forceinline__ float2 steering_weight_any(const double* p, const Ste
     const float2 v =
         cos_sin_turns((unsigned)__builtin_bit_cast(unsigned long long, r + 0x1.8p20));
     return make_float2(v.x + nan, v.y + nan);
+}
+
+// The weight in FP64, rounded once; a phase that is not finite gives NaN.
+__device__ __forceinline__ float2 steering_weight_exact(const double* p, const Steer& st) {
+    const double t = fma(p[2], st.d[2], fma(p[1], st.d[1], p[0] * st.d[0]));
+    const double2 v = cos_sin_turns64(t);
+    return make_float2((float)v.x, (float)v.y);
 }
 
 }  // namespace bfhip

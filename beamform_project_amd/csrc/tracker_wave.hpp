@@ -20,8 +20,8 @@
 // 16 cycles and some 53 other instructions, and the weights, about 43 a piece
 // (64 antennas, 672 channels, 65536 spectra, 32 beams, windows of 320: 1.85 ->
 // 1.34 ms, 0.54 PFLOP/s counted once; 13 beams, windows of 10, 4003 spectra,
-// 336 channels: 0.33 -> 0.23 ms; float weights instead of FP32 FMAs: 2 to 10
-// times faster).  Wave tasks run block, then channel fastest: a
+// 336 channels: 0.33 -> 0.23 ms; float weights there
+// instead of FP32 FMAs: 2.35 -> 0.41 ms).  Wave tasks run block, then channel fastest: a
 // workgroup's four waves read neighbouring channels (or the same one) of the
 // same spectra, which share 128-byte lines.
 //
@@ -30,8 +30,9 @@
 // Re(y_b) (weights wr, -wi), column 2b + 1 Im(y_b) (weights wi, wr).
 //
 // PARTS: weights as one fp16, as fp16 hi + lo (about 22 bits), or as three
-// bfloat16 slices that add up to the float (the FP32 selector).  Sums run
-// from the smallest slice to the largest.
+// bfloat16 slices that add up to the float (the FP32 selector), which then
+// comes from its own FP64 phase in every window.  Sums run from the smallest
+// slice to the largest.
 #pragma once
 
 #include <type_traits>
@@ -296,7 +297,11 @@ __device__ __forceinline__ void window_operands(const DirArgs& da, const BeamRow
             continue;
         }
         const Steer st = make_steer(d, ch.per_metre, ch.reach);
-        if (!anchored && __all(st.in_range)) {
+        if (PARTS == 3) {  // float weights: as exact as they are held
+            steps([&](int s, int jj) {
+                return steering_weight_exact(ch.pos.d + 3 * (a0 + 4 * s + 2 * jj), st);
+            });
+        } else if (!anchored && __all(st.in_range)) {
             steps([&](int s, int jj) {
                 return steering_weight_near(ch.pos.d + 3 * (a0 + 4 * s + 2 * jj), st);
             });
@@ -638,13 +643,15 @@ void launch_parts(hipStream_t stream, const TrackerLaunch& L, const DirArgs& da)
     constexpr int kMax2 = kMax < 2 ? kMax : 2;
     auto tasks = [&](size_t nt) { return ceil_div(L.B, nt * 8) * L.F * L.n_windows; };
     const bool two = kMax >= 2 && L.B > 8 && tasks(2) >= 2048;
-    if (L.S < (size_t)kDirectWeightMinSpectra) {
-        constexpr int kMaxAnchored = A * (PARTS + 1) <= 256 ? kMax2 : 1;
-        if (two && kMaxAnchored == 2)
-            launch_nt<A, kMaxAnchored, PARTS, INTEGRATE, true>(stream, L, da);
-        else
-            launch_nt<A, 1, PARTS, INTEGRATE, true>(stream, L, da);
-        return;
+    if constexpr (PARTS <= 2) {  // float weights are never rotated
+        if (L.S < (size_t)kDirectWeightMinSpectra) {
+            constexpr int kMaxAnchored = A * (PARTS + 1) <= 256 ? kMax2 : 1;
+            if (two && kMaxAnchored == 2)
+                launch_nt<A, kMaxAnchored, PARTS, INTEGRATE, true>(stream, L, da);
+            else
+                launch_nt<A, 1, PARTS, INTEGRATE, true>(stream, L, da);
+            return;
+        }
     }
     if (kMax >= 4 && L.B > 16 && tasks(4) >= 2048)
         launch_nt<A, kMax, PARTS, INTEGRATE, false>(stream, L, da);

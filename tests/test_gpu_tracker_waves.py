@@ -96,3 +96,32 @@ def test_direction_that_is_not_a_number(S):
     got[5:8, :, 3] = want[5:8, :, 3]
     got[17, :, 9] = want[17, :, 9]
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("A,S,antenna", [(32, 10, 9), (64, 10, 37), (64, 64, 22), (128, 16, 101),
+                                         (256, 80, 250)])
+def test_float_weights_are_rounded_once(A, S, antenna):
+    """The FP32 selector's weights are the FP64 phasor rounded to float, in
+    every window.  Two antennas see the same voltage 1, one at the origin and
+    one about half a turn away, phase pi + e with 2e-3 < e < 0.04: the power
+    (1 + wr)^2 + wi^2 is wi^2 to e^2 / 4.  One rounding of wi and those of its
+    square and the sum: 4 2^-24; 2^-25 in 1 + wr adds e^2 2^-25, 2^-25 of the
+    result.  An error of 2e-9 in the phase alone would be 1e-7 to 2e-6."""
+    F, B, W = 4, 9, 40
+    T = W * S
+    f0, l0 = 400e6, 0.25
+    fr = (f0 * (1 + 1e-3 * np.arange(F))).astype(np.float32)
+    pos = np.zeros((A, 3), np.float32)
+    pos[antenna, 0] = 0.5 * 299792458.0 / (f0 * l0)
+    # the phase's excess grows with channel, beam and window
+    l = l0 * (1 + 7e-4 * (1 + np.arange(B)) + 2e-5 * np.arange(W)[:, None])
+    dirs = np.stack([l, 0 * l, np.sqrt(1 - l * l)], -1).astype(np.float32)
+    x = np.zeros((T, F, A), np.uint8)
+    x[:, :, [0, antenna]] = 1
+    got = launch(x, pos, fr, dirs, T, F, A, B, S, False, K.FP32).reshape(W, S, F, B)
+    turns = pos[antenna, 0].astype(np.float64) * dirs[:, None, :, 0].astype(np.float64) * \
+        (fr.astype(np.float64) / 299792458.0)[None, :, None]
+    want = 4 * np.cos(np.pi * turns) ** 2  # [W][F][B]
+    assert np.all((want > 4e-6) & (want < 1.6e-3))
+    rel = np.abs(got / want[:, None] - 1)
+    assert rel.max() <= 4.5 * 2.0 ** -24, rel.max()
