@@ -196,6 +196,46 @@ __device__ __forceinline__ void load_float_weights(const float2* __restrict__ w,
     }
 }
 
+// Float weights may be infinite, and the zero samples past T turn that into a
+// NaN in a last window cut short by T.  Where such a window ended as a NaN, its
+// power is summed again over the rows it has, a row per lane (the result is an
+// infinity or a NaN: any order of sums gives it).  After the stages, by the
+// waves that stored the window: clearing the rows in the stage itself cost the
+// common path 10 registers and with them a wave per SIMD (A = 64, S = 10).
+template <int A, int NT>
+__device__ __noinline__ void repair_short_window(const uint8_t* __restrict__ x,
+                                                 const float2* __restrict__ w, bool tiled,
+                                                 float* __restrict__ out, int T, int F, int B,
+                                                 int S, int W, int f, int beam0, int lane) {
+    __threadfence_block();  // the window's stores, by other lanes of this wave
+    float* const o = out + ((size_t)(W - 1) * F + f) * B + beam0;
+    const int live = B - beam0 < NT * 8 ? B - beam0 : NT * 8;
+    unsigned long long bad = __ballot(lane < live && isnan(o[lane < live ? lane : 0]));
+    const int tiles = (B + 31) / 32;
+    while (bad != 0) {
+        const int i = __builtin_ctzll(bad);
+        bad &= bad - 1;
+        const int b = beam0 + i;
+        const float2* const wb = tiled ? w + ((size_t)f * tiles + b / 32) * A * 32 + b % 32
+                                       : w + ((size_t)b * F + f) * A;
+        float sum = 0.0f;
+        for (int t = (W - 1) * S + lane; t < T; t += kWaveSize) {
+            const uint8_t* const row = x + ((size_t)t * F + f) * A;
+            float re = 0.0f, im = 0.0f;
+            for (int a = 0; a < A; ++a) {
+                const float2 v = wb[a * (tiled ? 32 : 1)];
+                const float xr = (float)bf_nibble(row[a], 0), xi = (float)bf_nibble(row[a], 4);
+                re = fmaf(-v.y, xi, fmaf(v.x, xr, re));
+                im = fmaf(v.y, xr, fmaf(v.x, xi, im));
+            }
+            sum += re * re + im * im;
+        }
+#pragma unroll
+        for (int k = 32; k >= 1; k >>= 1) sum += __shfl_xor(sum, k);
+        if (lane == 0) o[i] = sum;
+    }
+}
+
 // At least two waves per SIMD (at most 256 registers per lane): the
 // unrolled stage otherwise keeps several tiles' accumulators in flight.
 template <int A, int NT, int WV, int PARTS, int MODE, int ST, bool DB, bool MASKED = false>
@@ -558,6 +598,9 @@ void mfma_fused_kernel(
             }
         }
     }
+    if constexpr (PARTS == 3 && MODE != 0)
+        if (has_beams && tile_end == tiles_total && T % S != 0)
+            repair_short_window<A, NT>(x, w, tiled, out, T, F, B, S, W, f, beam0, lane);
 }
 
 struct Plan {

@@ -98,3 +98,22 @@ def test_weights_outside_half_range():
     assert not np.isfinite(got[:, :, 1]).any()
     assert np.isnan(got[:, :, 2]).all() and np.isnan(got[:, :, 3]).all()
     assert np.isfinite(got[:, :, [0, 4, 5, 6, 7]]).all()
+
+
+@pytest.mark.parametrize("T,A,B,S", [(163, 64, 8, 10), (167, 64, 8, 12), (137, 64, 40, 20),
+                                     (203, 32, 17, 100), (171, 128, 9, 64), (330, 256, 9, 320),
+                                     (81, 256, 9, 16), (39, 64, 8, 10), (40, 64, 3, 7)])
+def test_infinite_weight_in_a_short_last_window(T, A, B, S):
+    """An infinite weight that every spectrum meets with a voltage of 1 + 1j
+    gives an infinite power in every window, a last one cut short by T too;
+    the other beams are as without it."""
+    x, w = random_case(T, A, B, seed=T + B)
+    w = w.reshape(B, F, A, 2).copy()
+    x[:, :, 7] = 0x11
+    dims = api.Dimensions(T, F, A, B)
+    want = run_gpu(K.FP32, x, w, dims, S)
+    w[1, :, 7] = (np.inf, 0.0)
+    got = run_gpu(K.FP32, x, w, dims, S)
+    assert np.isposinf(got[:, :, 1]).all()
+    got[:, :, 1] = want[:, :, 1]
+    assert np.array_equal(got, want)
