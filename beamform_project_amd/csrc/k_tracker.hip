@@ -273,7 +273,8 @@ void launch_tracker(hipStream_t stream, const TrackerLaunch& L) {
     const bool table = L.dir_source == kDirTable;
     const float* const q = L.trajectory;
     const DirArgs da{table ? L.dir_table : nullptr, table ? nullptr : L.trajectories,
-                     {q[0], q[1], q[2], q[3]}, (long)L.window_offset, (int)L.S, (int)L.B};
+                     {q[0], q[1], q[2], q[3]}, table ? 0L : (long)L.window_offset, (int)L.S,
+                     (int)L.B};
     if (!table && L.trajectories == nullptr && L.B != 1)
         invalid("a trajectory by value is for one beam");
     // One beam, per-spectrum output: the FP32 stream kernel (AUTO and FP32).

@@ -24,7 +24,7 @@ struct DirArgs {
     const float* table;  // directions [n_windows_table][B][3], or null for
     const float* traj;   // trajectories [B][4] = l0, m0, rate_l, rate_m, or null for
     float row[4];        // the only beam's trajectory
-    long window_offset;  // absolute index of local window 0
+    long window_offset;  // absolute index of local window 0; 0 with a table
     int S;
     int B;
 };

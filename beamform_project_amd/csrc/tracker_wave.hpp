@@ -168,17 +168,18 @@ __device__ __forceinline__ void slice_pair(float a, float b, unsigned (&out)[PAR
 // phase change delta = k (p . (d_w - d_anchor)), formed in FP32 from the
 // small direction difference (some 15 instructions instead of 38).  A beam
 // whose phases may have moved by 1/8 or more since its anchor is evaluated
-// from its own phase again.  Each window's weights depend only on w and its
-// anchor, never on how windows are grouped into launches.
+// from its own phase again.  On trajectories the index is the absolute one
+// (an anchor may lie before the launch's first window), so a window's weights
+// never depend on how windows are grouped into launches; a table holds the
+// launch's own windows only, and its anchors count from the launch's first.
 constexpr int kDirectWeightMinSpectra = 64;
-constexpr int kAnchorWindows = 16;
+constexpr int kAnchorWindows = 16;  // a power of two
 
 // Anchor phasors of this lane's own weights and the anchor's directions.
 template <int A, int NT>
 struct WeightAnchor {
     float2 own[NT][A / 16][2];
     float dir[NT][3];
-    int window = -1;  // none yet
 };
 
 // (cos, sin)(phi + delta) from z = (cos, sin)(phi), |delta| <= 1/8: the next
@@ -198,15 +199,17 @@ struct Channel {
     double per_metre;  // f / c
 };
 
-// B operand of one wave for window w.  Lane c holds column c of each 8-beam
+// B operand of one wave for window w, `since` windows after its anchor (`fresh`:
+// the anchor is not the one in `anc`).  Lane c holds column c of each 8-beam
 // N-tile (Re of beam c/2 for even c, Im for odd c) over the antennas
 // g (A/4) + 4 s + j.  Lanes c and c^1 need the same complex weights, so the
 // even lane evaluates j = 0, 2 and the odd lane j = 1, 3; each slices its own
 // and takes the partner's by DPP.
 template <int A, int NT, int PARTS, bool ANCHORED>
 __device__ __forceinline__ void window_operands(const DirArgs& da, const BeamRow (&rows)[NT],
-                                                const Channel<A>& ch, int w, int beam0, int lane,
-                                                bool direct, WeightAnchor<A, NT>& anc,
+                                                const Channel<A>& ch, int w, int since, bool fresh,
+                                                int beam0, int lane, bool direct,
+                                                WeightAnchor<A, NT>& anc,
                                                 bf_uint4v (&bw)[PARTS][NT][A / 16]) {
     constexpr int KS = A / 16;
     const int c = lane & 15;
@@ -215,7 +218,7 @@ __device__ __forceinline__ void window_operands(const DirArgs& da, const BeamRow
     const unsigned flip = odd ? 0u : 0x80008000u;
     const int a0 = g * (A / 4) + (odd ? 1 : 0);  // own antennas a0 + 4 s + 2 jj
     const bool anchored = ANCHORED && !direct;
-    const int wa = w - w % kAnchorWindows;
+    const int wa = w - since;
     // Direction of column c's beam.  Columns past the last beam hold the
     // weights of direction 0; they are not stored.
     auto direction = [&](int nt, int window, float (&d)[3]) {
@@ -223,7 +226,7 @@ __device__ __forceinline__ void window_operands(const DirArgs& da, const BeamRow
         d[0] = d[1] = d[2] = 0.0f;
         if (b < da.B) beam_direction(da, rows[nt], window, b, d);
     };
-    if (anchored && anc.window != wa) {
+    if (anchored && fresh) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             float d[3];
@@ -243,7 +246,6 @@ __device__ __forceinline__ void window_operands(const DirArgs& da, const BeamRow
             else
                 fill(steering_weight_any);
         }
-        anc.window = wa;
     }
     const float kf = (float)(kTwoPi * ch.per_metre);
 #pragma unroll
@@ -260,8 +262,8 @@ __device__ __forceinline__ void window_operands(const DirArgs& da, const BeamRow
                 dk[i] = kf * (d[i] - anc.dir[nt][i]);
                 bound += ch.reach[i] * fabsf(dk[i]);
             }
-            rotate = bound < 0.125f || (w == wa);
-            if (w == wa) dk[0] = dk[1] = dk[2] = 0.0f;
+            rotate = bound < 0.125f || since == 0;
+            if (since == 0) dk[0] = dk[1] = dk[2] = 0.0f;
         }
         // k-steps one after another, each with its weights from `make`; only
         // LDS reads may move across, which hides their latency (13 beams,
@@ -399,8 +401,9 @@ __device__ __forceinline__ void wave_windows(const RowSource& rs, const Channel<
     BeamRow rows[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) rows[nt] = beam_row(da, min(bl + 8 * nt, B - 1));
+    int since = ((int)da.window_offset + w_begin) & (kAnchorWindows - 1);
 #pragma unroll 1
-    for (int w = w_begin; w < w_end; ++w) {
+    for (int w = w_begin; w < w_end; ++w, since = (since + 1) & (kAnchorWindows - 1)) {
         const long t_win = rs.t_base + (long)w * S;
         auto load_tile = [&](int jt) -> TileBytes<A> {
             const long t0 = t_win + 16 * jt;
@@ -504,7 +507,9 @@ __device__ __forceinline__ void wave_windows(const RowSource& rs, const Channel<
             for (int u = 0; u < D; ++u)
                 if (u < tpw) buf[u] = load_tile(u);
         }
-        window_operands<A, NT, PARTS, ANCHORED>(da, rows, ch, w, beam0, lane, direct, anc, bw);
+        window_operands<A, NT, PARTS, ANCHORED>(da, rows, ch, w, since,
+                                                 since == 0 || w == w_begin, beam0, lane, direct,
+                                                 anc, bw);
         if (n_fast > 0) {
             bf_uint4v av[2][KS];
             auto group = [&](auto more, int j0) {

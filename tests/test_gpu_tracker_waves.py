@@ -125,3 +125,30 @@ def test_float_weights_are_rounded_once(A, S, antenna):
     assert np.all((want > 4e-6) & (want < 1.6e-3))
     rel = np.abs(got / want[:, None] - 1)
     assert rel.max() <= 4.5 * 2.0 ** -24, rel.max()
+
+
+@pytest.mark.parametrize("kernel", [K.SPLIT_F16, K.F16, K.FP32])
+@pytest.mark.parametrize("S", [10, 16, 64])
+def test_trajectory_windows_do_not_depend_on_the_launch(S, kernel):
+    """A run of windows on trajectories, whole and cut at windows that are and
+    are not multiples of an anchor's 16: the same bits."""
+    A, F, B, W = 64, 5, 11, 53
+    T = W * S
+    x, pos, fr, dirs = case(T, F, A, B, S, 4, step=1e-5)
+    rng = np.random.default_rng(8)
+    traj = np.concatenate([dirs[0, :, :2], rng.uniform(-2e-6, 2e-6, (B, 2))], 1).astype(np.float32)
+    dpos, dfr, dtraj = [api.DeviceArray.from_numpy(a) for a in (pos, fr, traj)]
+
+    def part(first, last):
+        dx = api.DeviceArray.from_numpy(np.ascontiguousarray(x[first * S:last * S]))
+        out = api.DeviceArray.empty((last - first, F, B), np.float32)
+        TR.multibeam_tracker_launch(None, dx, out, (last - first) * S, F, A, B, S, dpos, dfr,
+                                    trajectories=dtraj, window_offset=first, integrate=True,
+                                    kernel=kernel)
+        api.device_synchronize()
+        return out.to_numpy()
+
+    whole = part(0, W)
+    for cuts in ([0, 7, 8, 30, W], [0, 16, 48, W], [0, 1, 33, 47, W]):
+        got = np.concatenate([part(a, b) for a, b in zip(cuts, cuts[1:])])
+        assert np.array_equal(got, whole), cuts
