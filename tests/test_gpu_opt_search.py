@@ -1,5 +1,7 @@
 """The adaptive search at the sizes where its batches, blocks and tiles end:
-runs of 1 to 10 windows (batches of 1, then 4), a short last window, steered
+runs of 1 to 25 windows (batches of 1, 2, 4 and then 8 windows in two slots: the
+fourth batch is the first to fill a slot, the fifth to use one the third time), a
+short last window, steered
 antennas around blocks of 16, coarse grids below, at and above one tile of 16
 cells and above one pass of the reduction, with and without refinement and
 forgetting, one channel group and many.  Against the oracle's restatement in
@@ -23,6 +25,7 @@ pytestmark = pytest.mark.gpu
     (64, 140, 70, 9, 2, 49, 0.6, 0), (32, 90, 9, 4, 2, 31, 0.9, 0),
     (32, 250, 50, 5, 2, 0, 0.9, 1), (32, 130, 60, 4, 1, 16, 0.5, 1),
     (64, 650, 70, 6, 2, 0, 0.9, 1), (64, 200, 100, 23, 0, 48, 1.0, 1),
+    (32, 220, 9, 4, 1, 0, 0.9, 0), (32, 982, 40, 4, 1, 0, 0.9, 1),
 ])
 def test_search_matches_restatement(A, T, S, G, levels, p_sub, lam, estimator):
     pos, fr = O.default_positions(A), O.channelized_frequencies(F)
