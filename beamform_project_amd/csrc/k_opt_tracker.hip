@@ -385,8 +385,8 @@ struct ScanTypes<double> {
     __device__ static int antenna(int j, int r, int g) { return 16 * j + 4 * r + g; }
 };
 
-// This lane's part of sum_I [...] over the block rows I = i0, i1 (i1 < 0: all
-// rows from i0) of the cell whose phase per metre (in turns) is d.
+// This lane's part of sum_I [...] over the block rows I whose bit is set in
+// `rows`, for the cell whose phase per metre (in turns) is d.
 template <typename T>
 __device__ __forceinline__ T scan_form(const T* __restrict__ X, int Mp, const double* s_pos,
                                        const double (&d)[3], unsigned rows, int lane) {
@@ -456,13 +456,13 @@ __device__ void decide(const ScanArgs& a, float* P, double* sums, OptSearch* out
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int n_cells = a.before_cells;
-    const int groups = a.before_groups;
+    const DecideSplit d = decide_split(n_cells, a.before_groups);
     const int level = a.before_level, last_level = a.last_level;
     const OptGridArgs& g = a.g;
-    decide_sum(tid, n_cells, groups, a.before_part, P, sums);
+    decide_sum(d, tid, n_cells, a.before_groups, a.before_part, P, sums);
     __syncthreads();
-    if (decide_split(n_cells, groups).ways > 1) {
-        decide_fold(tid, n_cells, groups, sums, P);
+    if (d.ways > 1) {
+        decide_fold(d, tid, n_cells, sums, P);
         __syncthreads();
     }
     if (tid >= 64) return;

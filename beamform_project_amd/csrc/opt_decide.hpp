@@ -33,9 +33,8 @@ BF_HOST_DEVICE DecideSplit decide_split(int n_cells, int groups) {
 
 // Thread `tid`'s sums, in FP64 and a fixed order: with several ways into
 // sums[kScanThreads], else into P[n_cells], which holds no padding.
-BF_HOST_DEVICE void decide_sum(int tid, int n_cells, int groups, const double* part, float* P,
-                               double* sums) {
-    const DecideSplit d = decide_split(n_cells, groups);
+BF_HOST_DEVICE void decide_sum(const DecideSplit& d, int tid, int n_cells, int groups,
+                               const double* part, float* P, double* sums) {
     for (int i = tid; i < d.padded * d.ways; i += kScanThreads) {
         const int cell = i % d.padded, way = i / d.padded;
         const int last = (way + 1) * d.per;
@@ -51,8 +50,8 @@ BF_HOST_DEVICE void decide_sum(int tid, int n_cells, int groups, const double* p
 }
 
 // Where several ways shared a cell (after a barrier): thread `tid`'s cells.
-BF_HOST_DEVICE void decide_fold(int tid, int n_cells, int groups, const double* sums, float* P) {
-    const DecideSplit d = decide_split(n_cells, groups);
+BF_HOST_DEVICE void decide_fold(const DecideSplit& d, int tid, int n_cells, const double* sums,
+                                float* P) {
     for (int cell = tid; cell < n_cells; cell += kScanThreads) {
         double sum = 0.0;
         for (int way = 0; way < d.ways; ++way) sum += sums[way * d.padded + cell];

@@ -16,11 +16,12 @@ static int check(int n_cells, int groups) {
     const float kUnwritten = -1.0f;
     std::vector<float> P(n_cells + 64, kUnwritten);
     std::vector<double> sums(kScanThreads + 64, kUnwritten);
+    const DecideSplit d = decide_split(n_cells, groups);
     for (int t = 0; t < kScanThreads; ++t)
-        decide_sum(t, n_cells, groups, part.data(), P.data(), sums.data());
-    if (decide_split(n_cells, groups).ways > 1)
+        decide_sum(d, t, n_cells, groups, part.data(), P.data(), sums.data());
+    if (d.ways > 1)
         for (int t = 0; t < kScanThreads; ++t)
-            decide_fold(t, n_cells, groups, sums.data(), P.data());
+            decide_fold(d, t, n_cells, sums.data(), P.data());
     int bad = 0;
     for (int i = 0; i < 64; ++i)
         bad += P[n_cells + i] != kUnwritten || sums[kScanThreads + i] != kUnwritten;
