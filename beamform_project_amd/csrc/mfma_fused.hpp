@@ -238,7 +238,10 @@ __device__ __noinline__ void repair_short_window(const uint8_t* __restrict__ x,
 
 // At least two waves per SIMD (at most 256 registers per lane): the
 // unrolled stage otherwise keeps several tiles' accumulators in flight.
-template <int A, int NT, int WV, int PARTS, int MODE, int ST, bool DB, bool MASKED = false>
+// SHORT: float weights and a last window cut short by T (a kernel of its own:
+// the check alone cost whole windows 2 %).
+template <int A, int NT, int WV, int PARTS, int MODE, int ST, bool DB, bool MASKED = false,
+          bool SHORT = false>
 __global__ __launch_bounds__(WV * kWaveSize) __attribute__((amdgpu_waves_per_eu(2)))
 void mfma_fused_kernel(
     const uint8_t* __restrict__ x, const float2* __restrict__ w, bool tiled,
@@ -598,8 +601,8 @@ void mfma_fused_kernel(
             }
         }
     }
-    if constexpr (PARTS == 3 && MODE != 0)
-        if (has_beams && tile_end == tiles_total && T % S != 0)
+    if constexpr (SHORT)
+        if (has_beams && tile_end == tiles_total)
             repair_short_window<A, NT>(x, w, tiled, out, T, F, B, S, W, f, beam0, lane);
 }
 
@@ -719,11 +722,17 @@ void launch_shape(hipStream_t stream, const MfmaLaunch& L, const MfmaConfig& cfg
     const dim3 grid((unsigned)(p.per_xcd * kXcds), (unsigned)p.beam_blocks);
     const dim3 block(WV * kWaveSize);
     const float2* w2 = reinterpret_cast<const float2*>(L.w);
-#define BF_LAUNCH(MODE_, ST_)                                                                 \
-    hipLaunchKernelGGL((mfma_fused_kernel<A, NT, WV, PARTS, MODE_, ST_, DB, MASKED>), grid,   \
-                       block, 0,                                                               \
-                       stream, L.x, w2, L.tiled, L.out, L.mask, L.T, L.F, L.B, L.S, p.W,       \
-                       p.tiles_total, p.tiles_per_chunk, p.n_items, p.per_xcd)
+#define BF_LAUNCH_SHORT(MODE_, ST_, SHORT_)                                                     \
+    hipLaunchKernelGGL((mfma_fused_kernel<A, NT, WV, PARTS, MODE_, ST_, DB, MASKED, SHORT_>),   \
+                       grid, block, 0, stream, L.x, w2, L.tiled, L.out, L.mask, L.T, L.F, L.B,  \
+                       L.S, p.W, p.tiles_total, p.tiles_per_chunk, p.n_items, p.per_xcd)
+#define BF_LAUNCH(MODE_, ST_)                                     \
+    do {                                                          \
+        if (PARTS == 3 && MODE_ != 0 && L.T % L.S != 0)           \
+            BF_LAUNCH_SHORT(MODE_, ST_, PARTS == 3 && MODE_ != 0); \
+        else                                                      \
+            BF_LAUNCH_SHORT(MODE_, ST_, false);                   \
+    } while (0)
     if (p.mode == 0) {
         BF_LAUNCH(0, 4);
     } else if (p.mode == 1) {
@@ -738,6 +747,7 @@ void launch_shape(hipStream_t stream, const MfmaLaunch& L, const MfmaConfig& cfg
         BF_LAUNCH(2, 1);
     }
 #undef BF_LAUNCH
+#undef BF_LAUNCH_SHORT
 }
 
 template <int A, int NT, int WV>
