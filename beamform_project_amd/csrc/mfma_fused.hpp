@@ -205,7 +205,7 @@ __device__ __forceinline__ void load_float_weights(const float2* __restrict__ w,
 template <int A, int NT>
 __device__ __noinline__ void repair_short_window(const uint8_t* __restrict__ x,
                                                  const float2* __restrict__ w, bool tiled,
-                                                 float* __restrict__ out, int T, int F, int B,
+                                                 float* out, int T, int F, int B,
                                                  int S, int W, int f, int beam0, int lane) {
     __threadfence_block();  // the window's stores, by other lanes of this wave
     float* const o = out + ((size_t)(W - 1) * F + f) * B + beam0;

@@ -20,10 +20,10 @@
 // 16 cycles and some 53 other instructions, and the weights, about 43 a piece
 // (64 antennas, 672 channels, 65536 spectra, 32 beams, windows of 320: 1.85 ->
 // 1.34 ms, 0.54 PFLOP/s counted once; 13 beams, windows of 10, 4003 spectra,
-// 336 channels: 0.33 -> 0.23 ms; float weights there
-// instead of FP32 FMAs: 2.35 -> 0.41 ms).  Wave tasks run block, then channel fastest: a
-// workgroup's four waves read neighbouring channels (or the same one) of the
-// same spectra, which share 128-byte lines.
+// 336 channels: 0.33 -> 0.20 ms; float weights there, 2.35 ms on FP32 FMAs,
+// 0.41 ms).  Wave tasks run block, then channel fastest: a workgroup's four waves
+// read neighbouring channels (or the same one) of the same spectra, which share
+// 128-byte lines.
 //
 // Element order within a lane's 8 contraction slots: (re0, re2, im0, im2,
 // re1, re3, im1, im3) of antennas 0..3 of a dword; output column 2b holds

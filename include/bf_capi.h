@@ -72,11 +72,13 @@ bf_status bf_quantization_parameter_count(const bf_dims* integrated_dims, size_t
 /* ----------------------------------------------------- kernel choice */
 /* Reference: include/beamformer/cuda_stage_api.hpp:14-17
  * (CudaBeamformerKernel {Direct, Tiled}).  DIRECT reads canonical weights,
- * TILED the tiled layout; both run the plain FP32 fused kernel and keep the
+ * TILED the tiled layout; both take float weights as FP32 does and keep the
  * reference's integration rules (Direct: 320 only; Tiled: 10 or 320).
  * The remaining selectors are additions of this build; all take canonical
  * weights and accept any integration_spectra >= 1:
- *   FP32       plain FP32 fused kernel (VALU FMA)
+ *   FP32       float weights, FP32 accumulate: on the matrix cores as three
+ *              bfloat16 slices that add up to the weight, small calls and
+ *              other window lengths on FP32 FMAs
  *   SPLIT_F16  FP16 MFMA, weights split hi+lo, FP32 accumulate (~FP32 accuracy)
  *   F16        FP16 MFMA, single FP16 weights (~1e-3 relative)
  *   AUTO       SPLIT_F16 where supported, else FP32 */
