@@ -615,17 +615,19 @@ struct Plan {
 // at a time instead of one: fewer barriers per tile, five times the LDS.  Up
 // to 64 antennas that is free (split, S = 20, T = 4100, B = 33: A = 32 69 -> 38
 // us, A = 64 73 -> 61 us).  Above it leaves two workgroups to a CU, which
-// costs nothing where no more were launched (A = 128, T = 512, B = 9, S = 20, 336
-// workgroups: 32 -> 27 us; S = 40, 672 of them: 35 -> 41 us).  Beyond those it
-// pays at 128 for two N-tiles of split weights (T = 4100, B = 33, S = 100: 180
-// -> 141 us; but B = 2 87 -> 112 us, F16 98 -> 106 us) and at 256 in long
-// calls (T = 4100, S = 100, B = 33: 510 -> 448 us; T = 1024, B = 20: 71 -> 80 us), for
-// single weights with one block of beams (T = 4100, S = 20: B = 9 0.88 of the
-// time, B = 33 1.05).  Float weights were measured with five tiles only.
-inline bool five_tile_stages(int A, int parts, int nt, int T, int B, long workgroups) {
-    if (A <= 64 || parts == 3 || workgroups <= 512) return true;
-    if (A == 128) return parts == 2 && nt >= 2;
-    return T >= 4096 && (parts == 2 || B <= 32);
+// costs nothing where no more were launched and there are stages to overlap
+// (A = 128, T = 512, B = 9, S = 20, 336 workgroups of 35 tiles: 32 -> 27 us; S = 40,
+// 672 of them: 35 -> 41 us; A = 256, S = 100, T = 65, B = 20, 25 tiles: 34 -> 31 us; but
+// S = 60, T = 200, 15 tiles 25 -> 29 us, and A = 128, S = 20, T = 70, B = 40, 5 tiles 12.8
+// -> 13.7 us).  Beyond those it pays at 128 for two N-tiles of split weights (T =
+// 4100, B = 33, S = 100: 180 -> 141 us; but B = 2 87 -> 112 us, F16 98 -> 106 us) and
+// at 256 in long calls (T = 4100, S = 100, B = 33: 510 -> 448 us; T = 1024, B = 20: 71
+// -> 80 us), for single weights with one block of beams (T = 4100, S = 20: B = 9
+// 0.88 of the time, B = 33 1.05).  Float weights were measured with five tiles only.
+inline bool five_tile_stages(int A, int parts, int nt, int T, int B, long workgroups, int tiles) {
+    if (A <= 64 || parts == 3) return true;
+    if (A == 128) return tiles > 5 && (workgroups <= 512 || (parts == 2 && nt >= 2));
+    return (workgroups <= 512 && tiles >= 25) || (T >= 4096 && (parts == 2 || B <= 32));
 }
 
 inline Plan make_plan(int A, int parts, int T, int F, int B, int S, bool one_by_one,
@@ -685,7 +687,7 @@ inline Plan make_plan(int A, int parts, int T, int F, int B, int S, bool one_by_
     p.n_items = n_chunks * F;
     p.per_xcd = (int)ceil_div((size_t)p.n_items, kXcds);
     if (p.mode == 2 && p.st == 1 && tiles_per_super % 5 == 0 &&
-        five_tile_stages(A, parts, cfg.nt, T, B, (long)p.n_items * p.beam_blocks))
+        five_tile_stages(A, parts, cfg.nt, T, B, (long)p.n_items * p.beam_blocks, per_chunk))
         p.st = 5;
     return p;
 }
