@@ -622,13 +622,12 @@ template <int A, int NT, int PARTS, bool INTEGRATE, bool ANCHORED>
 void launch_nt(hipStream_t stream, const TrackerLaunch& L, const DirArgs& da) {
     const size_t tpw = ceil_div(L.S, 16);
     const size_t blocks = ceil_div(L.B, (size_t)(NT * 8));
-    // Windows per task: about 32 tiles, or an anchor's 16 windows as long as
-    // two waves per SIMD remain.
-    size_t run = ceil_div(32, tpw);
-    if (ANCHORED) {
-        run = kAnchorWindows;
+    // Windows per task: about 32 tiles, or an anchor's 16 windows; short windows
+    // as long as two waves per SIMD remain (float weights, 32 antennas, 17
+    // channels, 200 spectra, 3 beams, windows of 10: 32 tiles 32 us, this 10 us).
+    size_t run = ANCHORED ? kAnchorWindows : ceil_div(32, tpw);
+    if (L.S < (size_t)kDirectWeightMinSpectra)
         while (run > 1 && ceil_div(L.n_windows, run) * L.F * blocks < 2048) run /= 2;
-    }
     const size_t n_tasks = ceil_div(L.n_windows, run) * L.F * blocks;
     const size_t per_xcd = ceil_div(ceil_div(n_tasks, kWaves), kXcds);
     if (per_xcd * kXcds > (size_t)INT32_MAX)
